@@ -169,7 +169,10 @@ int ssq_device_cus();
 // grid-search encode (ssq_encode_grid.hip)
 bool ssq_encode_grid_supported(const ssq_encode_args* a);
 int ssq_encode_grid_run(const ssq_encode_args* a, hipStream_t st);
-// exact encode for codebooks of more than 256 codewords (ssq_encode_wide.hip)
+// matrix-core screen + exact evaluation (ssq_encode_tile.hip): 256 codewords, or more than 256 with
+// block dims up to 8
+int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st);
+// exact scan for codebooks of more than 256 codewords (ssq_encode_wide.hip)
 int ssq_encode_wide_run(const ssq_encode_args* a, hipStream_t st);
 
 #define SSQ_REQUIRE(cond, ...)                                  \

@@ -70,4 +70,11 @@ __device__ __forceinline__ void out_rows(const ssq_encode_args& a, int b, int kv
     }
 }
 
+// code element i (in units of the code width) of a row buffer
+__device__ __forceinline__ void store_code(uint8_t* codes, int width, int64_t i, uint32_t v) {
+    if (width == 1) codes[i] = (uint8_t)v;
+    else if (width == 2) reinterpret_cast<uint16_t*>(codes)[i] = (uint16_t)v;
+    else reinterpret_cast<uint32_t*>(codes)[i] = v;
+}
+
 }  // namespace

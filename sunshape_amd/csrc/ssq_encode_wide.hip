@@ -30,11 +30,6 @@ struct WideEncodeParams {
     int vec;      // 1: each codeword row is 4 * block_dim-byte aligned (vector staging loads)
 };
 
-__device__ __forceinline__ void store_code(uint8_t* codes, int width, int64_t i, uint32_t v) {
-    if (width == 2) reinterpret_cast<uint16_t*>(codes)[i] = (uint16_t)v;
-    else reinterpret_cast<uint32_t*>(codes)[i] = v;
-}
-
 // one codeword's pre-sqrt distance v (not yet clamped)
 template <int BD, bool MM>
 __device__ __forceinline__ float stage_dist(const float* x, float xn, const float* cb, const float* cn, int j, int bd) {
