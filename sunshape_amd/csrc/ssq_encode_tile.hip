@@ -1,5 +1,5 @@
 // Nearest-codeword encode on the matrix cores (SunShapeBlockCodec.quantize, sunshape/codec.py:362-385):
-// a bf16 MFMA screen finds, per (key, block), the one group of 8 codewords that can hold the
+// a bf16 MFMA screen finds, per (key, block), the one group of 8 or 16 codewords that can hold the
 // reference's winner, and the reference's own fp32 arithmetic decides inside it.  Serves 256-codeword
 // codebooks (kernel 2) and, with the codebook streamed through LDS, codebooks past 256 codewords.
 //
@@ -8,20 +8,27 @@
 // Every fp32 number enters as a sum of bf16 parts (RNE, each the rounding of what the previous left):
 //   bf16 keys (and fp32 keys whose low halves are all zero):  x . (c_hi + c_mid + c_lo), exact products;
 //   other keys:  x_hi (c_hi + c_mid) + x_mid c_hi, which leaves out at most 3 2^-18 |x||c| per product;
+//   block dims 1 and 2, any key:  the six products down to 2^-18, which leave out less than 2^-25 |x||c|;
 //   |c|^2 in three parts against 1, X_up against 1.
-// That is 3 bd + 4 of the K slots: one MFMA for block dims up to 4, two for 8, four for 16.  v_j >= 0
-// up to rounding, so its bits order as a signed int.
+// That is 3 bd + 4 (6 bd + 4) of the K slots: one MFMA for block dims up to 4, two for 8, four for 16.
+// v_j >= 0 up to rounding, so its bits order as a signed int.
 //
 // What it replaces and why.  The fp32 form (v_mfma_f32_16x16x4f32, K = bd + 2 padded to 8) spent 64
 // matrix-core cycles per 256 distances and three VALU instructions per distance on the lane's two
 // smallest values.  Here a 32x32 tile takes 32 cycles per 1,024 distances, and the VALU takes
-// v_min3_i32 over each group of 8 codewords before the tagged (min, second min) pair sees it: 7
-// instructions per 8 distances.  The exact evaluation then takes 4 codewords per lane (8 past 256
-// codewords) for each (key, block).
+// v_min3_i32 over each group of 8 codewords (16 past 256 codewords) before the tagged (min, second
+// min) pair sees it: 7 instructions per 8 distances (11 per 16).  The exact evaluation then takes half
+// a group on each of a key's two lanes.
 //
-// Error bound.  P_j = (|x| + |c_j|)^2.  The 3 bd + 4 terms of v_j pass through at most that many
+// Measured, one MI355X, the fp32 screen / exact scan before -> this kernel: 262,144 bf16 keys of head_dim
+// 128 at block_dim 4, 256 codewords: 625 -> 164 us (77 MB, 15 us at a copy's rate: VALU issue bounds it,
+// 288 VALU instructions per 32 keys and block at 73 % issue, the matrix cores 13 % busy); 65,536 fp32
+// keys at 4,096 codewords of dim 4: 1,448 -> 375 us; a 64-sequence decode step's append: unchanged,
+// 11 us.
+//
+// Error bound.  P_j = (|x| + |c_j|)^2.  The terms of v_j pass through at most as many
 // roundings (any order, even truncation) of partial sums of at most 1.02 P_j, |c_j|^2 carries the
-// bd roundings of the reference's own norm, and the parts left out of a two-part key add 1.53 2^-18 P_j:
+// bd roundings of the reference's own norm, and the parts left out add 1.53 2^-18 P_j (2^-24):
 // |v_j - (|x - c_j|^2 + X_up - |x|^2)| <= A P_j.  The reference's chain r_j is within g P_j of
 // |x - c_j|^2, g = 1.001 (bd + 2) 2^-23.  With |c_j| <= |x| + |x - c_j|, P_j <= 6 |x|^2 + 3 |x - c_j|^2.
 // The reference's winner j* has sqrt(r_j*) <= sqrt(r_m) for the screen's minimum m, and a correctly
@@ -57,7 +64,13 @@ constexpr int kTileThreads = kTileWaves * SSQ_WAVE;
 constexpr int kTileKeys = kTileWaves * 32;
 // keys per slot of the staged keys, padded by one: consecutive slots then start two banks apart
 constexpr int kKeyRow = kTileKeys + 1;
-constexpr int kStageCw = 256;  // codewords per LDS stage: 8 tiles of 32
+// Codewords per group: 8 where each block of 256 pays for the exact evaluation of a group; 16 past
+// that, where the screen is nearly all of it (11 instructions per 16 distances instead of 14).
+constexpr int group_cw(bool wide) { return wide ? 16 : 8; }
+// tiles per (min, second min) pair: 16 group tags
+constexpr int tag_tiles(bool wide) { return group_cw(wide); }
+// codewords per LDS stage: a 256-codeword block, or 1,024 (block dim 8: 512) codewords of a longer one
+constexpr int stage_cw(int bdp, bool wide) { return !wide ? 256 : bdp <= 4 ? 1024 : 512; }
 constexpr size_t kTileSmemCap = 160 * 1024;
 constexpr int kMaxLightTile = 128;
 
@@ -71,32 +84,46 @@ struct TileParams {
     int xg, groups;      // key groups per (sequence, KV head), and in all
     int row_codes;       // 1: one chunk holds every light block and code rows take 16-byte stores
     int vec;             // 1: codeword rows are aligned for vector loads
+    int pieces;          // 16-byte pieces per key row where rows load whole (a power of two), else 0
     uint8_t light[kMaxLightTile];  // light (VQ-coded) block ids, ascending
 };
 
-template <int BDP>
+template <int BDP, bool WIDE>
 struct TileShape {
-    static constexpr int NM = (3 * BDP + 4 + 15) / 16;        // MFMAs per tile
-    static constexpr int kOps = 8 * NM * 256;                 // dwords of one stage's codeword operand
-    static constexpr int kRec = 4 * BDP + 4;                  // 4 codewords and their norms (dwords)
-    static constexpr int kRecs = (kStageCw / 4) * kRec;
+    static constexpr int kNorm = BDP == 2 ? 6 : 3 * BDP / 2;         // operand dword of the norm's parts
+    static constexpr int NM = (2 * (kNorm + 2) + 15) / 16;           // MFMAs per tile
+    static constexpr int kTiles = stage_cw(BDP, WIDE) / 32;
+    static constexpr int kOps = kTiles * NM * 256;                   // dwords of one stage's codeword operand
+    static constexpr int kRec = 4 * BDP + 4;                         // 4 codewords and their norms (dwords)
+    static constexpr int kRecs = WIDE ? 0 : stage_cw(BDP, WIDE) / 4 * kRec;
 };
 constexpr int slot_dwords(int bdp, bool raw16) { return raw16 ? bdp / 2 : bdp; }
 
-// LDS: operands [2][kOps] | (one stage only: records [2][kRecs]) | bad [nbc], two-part flag | slot of
-//      block [128] | heavy blocks [128] | keys [nbc][kKeyRow][slot dwords]
-template <int BDP>
-size_t tile_smem(int nbc, bool raw16, bool wide) {
-    using Sh = TileShape<BDP>;
-    size_t dw = 2 * (size_t)Sh::kOps + (wide ? 0 : 2 * (size_t)Sh::kRecs) + (size_t)((nbc + 4) & ~3) + 64;
-    return (dw + (size_t)nbc * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
+// (key, block) pairs a workgroup can put off to its end (the full scans); more are scanned at once
+constexpr int kOpenCap = 512;
+
+// LDS: operands [2][kOps] | (one stage only: records [2][kRecs]) | bad [nbc], two-part flag, open
+//      count | slot of block [128] | heavy blocks [128] | open pairs [kOpenCap] u16 | keys [nbc + 1][kKeyRow][slot dwords] (the last slot takes
+//      the dims of other chunks and of heavy blocks where rows load whole; block dims 9 and 10 are
+//      always gathered and have none)
+template <int BDP, bool WIDE>
+size_t tile_smem(int nbc, bool raw16) {
+    using Sh = TileShape<BDP, WIDE>;
+    const size_t dw = 2 * (size_t)Sh::kOps + 2 * (size_t)Sh::kRecs + (size_t)((nbc + 5) & ~3) + 64 + kOpenCap / 2;
+    return (dw + (size_t)(nbc + (BDP < 16 ? 1 : 0)) * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
 }
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
     const v2f f = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf));
 }
-__device__ __forceinline__ float bf16_round(float a) { return (float)(__bf16)a; }
+// both values' bf16 roundings, packed, and what they leave
+__device__ __forceinline__ uint32_t split2(float v0, float v1, float& r0, float& r1) {
+    const uint32_t w = pk_bf16(v0, v1);
+    r0 = v0 - __uint_as_float(w << 16);
+    r1 = v1 - __uint_as_float(w & 0xFFFF0000u);
+    return w;
+}
 
 // this lane's value and that of the lane 32 apart, in an order that differs between the two: only
 // symmetric combinations are taken
@@ -130,7 +157,7 @@ __device__ __forceinline__ float exact_e(const float (&m2x)[BDP], float xn, cons
     for (int d = 1; d < BDP; ++d) acc = __builtin_fmaf(m2x[d], c[d], acc);
     acc = __builtin_fmaf(xn, 1.0f, acc);
     acc = __builtin_fmaf(1.0f, cn, acc);
-    return acc > 0.f ? acc : 0.f;
+    return fmaxf(acc, 0.f);
 }
 
 // the two smallest of a set of clamped distances (as their bits: values >= 0 order like ints), and
@@ -182,8 +209,8 @@ __device__ __forceinline__ void slot_elems(const uint32_t (&w)[slot_dwords(BDP, 
 
 // the codeword row j of a block (zero-padded to BDP), in the metric space when met is given
 template <int BDP>
-__device__ __forceinline__ void load_row(const float* cent, int64_t j, int bd, int vec, float (&c)[BDP]) {
-    const float* s = cent + j * bd;
+__device__ __forceinline__ void load_row(const float* cent, uint32_t j, int bd, int vec, float (&c)[BDP]) {
+    const float* s = cent + j * (uint32_t)bd;  // at most 2^20 rows of 16: a 32-bit offset from a uniform base
     if (vec) {  // bd == BDP
         if constexpr (BDP == 2) {
             const float2 v = *reinterpret_cast<const float2*>(s);
@@ -232,8 +259,8 @@ __device__ __forceinline__ void wave_sync_lds() {
 // stage of codewords per block.
 template <int BDP, int KM, bool WIDE>
 __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p) {
-    using Sh = TileShape<BDP>;
-    constexpr int NM = Sh::NM;
+    using Sh = TileShape<BDP, WIDE>;
+    constexpr int NM = Sh::NM, kNorm = Sh::kNorm, kGc = group_cw(WIDE), kTagTiles = tag_tiles(WIDE);
     constexpr int SD = slot_dwords(BDP, KM != kKeyF32);
     extern __shared__ __align__(16) uint32_t tile_lds[];
     const ssq_encode_args& a = p.a;
@@ -260,14 +287,16 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
 
     u32a* ops = tile_lds;
     u32a* recs = ops + 2 * Sh::kOps;
-    u32a* bad = recs + (WIDE ? 0 : 2 * Sh::kRecs);
+    u32a* bad = recs + 2 * Sh::kRecs;
     u32a* two_part = bad + p.nbc;
-    uint8_t* blkslot = reinterpret_cast<uint8_t*>(bad + ((p.nbc + 4) & ~3));
+    uint32_t* n_open = tile_lds + 2 * Sh::kOps + 2 * Sh::kRecs + p.nbc + 1;
+    uint8_t* blkslot = reinterpret_cast<uint8_t*>(bad + ((p.nbc + 5) & ~3));
     uint8_t* heavyL = blkslot + 128;
-    u32a* keysL = reinterpret_cast<u32a*>(heavyL + 128);
+    u16a* open_list = reinterpret_cast<u16a*>(heavyL + 128);
+    u32a* keysL = reinterpret_cast<u32a*>(open_list + kOpenCap);
     u32a* mykeys = keysL + (wave * 32) * SD;  // slot j of key m: mykeys + (j * kKeyRow + m) * SD
 
-    for (int j = tid; j <= p.nbc; j += kTileThreads) bad[j] = 0;  // and *two_part
+    for (int j = tid; j <= p.nbc + 1; j += kTileThreads) bad[j] = 0;  // and *two_part, *n_open
     if (tid < nb) {
         const bool hv = ssq_is_heavy(hm0, hm1, tid);
         const int ho = heavy_ordinal(hm0, hm1, tid);
@@ -289,13 +318,80 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         out_rows(a, b, kv, s, crow, prow);
     }
 
-    // keys -> LDS, permuted: slot j holds light block l0 + j's elements.  A lane takes one element
-    // position (its dim comes from the permutation once) of 64 / epad keys at a time; the lanes of a
-    // key gather inside its row.
+    // keys -> LDS, permuted: slot j holds light block l0 + j's elements.
+    //  Whole rows: each lane loads 16-byte pieces of several keys, always the same dims, and scatters
+    //  the elements to the byte offsets the inverse permutation gives for those dims (an LDS table,
+    //  in the operand buffers' space): no arithmetic per element.
+    //  Otherwise (unaligned rows, padded block dims, a permutation that repeats a dim): a lane takes
+    //  one element position, its dim from the permutation, of 64 / epad keys at a time.
     uint32_t low = 0;  // any nonzero low half of an fp32 element
+    const int E = nl * BDP;
+    int pieces = p.pieces;
+    if (pieces) {  // uniform
+        constexpr int kElem = KM == kKeyF32 ? 4 : 2;
+        constexpr int N = 8;  // pieces in flight per lane; the first ones load while the table is built
+        uint4 v[N];
+        const int pc = lane & (pieces - 1), m0 = lane / pieces, kpl = 64 / pieces, n_loads = pieces / 2;
+        auto load_pieces = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int m = min(i0 + i, n_loads - 1) * kpl + m0;
+                const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)krow, m);
+                const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)((uint64_t)krow >> 32), m);
+                const int64_t row = (int64_t)(((uint64_t)hi << 32) | lo);
+                v[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(a.keys) + row * kElem + pc * 16);
+            }
+        };
+        if (live) load_pieces(0);
+        const uint32_t other = (uint32_t)(p.nbc * kKeyRow * SD * 4);
+        for (int d = tid; d < D; d += kTileThreads) ops[d] = other;
+        __syncthreads();  // also: bad and *two_part are cleared
+        auto dim_of = [&](int e) { return (int)perm[p.light[l0 + e / BDP] * bd + e % BDP]; };
+        auto off_of = [&](int e) { return (uint32_t)((e / BDP) * kKeyRow * SD * 4 + (e % BDP) * kElem); };
+        for (int e = tid; e < E; e += kTileThreads) {
+            const int dim = dim_of(e);
+            if ((unsigned)dim < (unsigned)D) ops[dim] = off_of(e);
+        }
+        __syncthreads();
+        for (int e = tid; e < E; e += kTileThreads) {
+            const int dim = dim_of(e);
+            if ((unsigned)dim >= (unsigned)D || ops[dim] != off_of(e)) *two_part = 2;  // a dim twice
+        }
+        __syncthreads();
+        const bool twice = *two_part == 2;
+        constexpr int kPer = 16 / kElem;  // elements per piece
+        uint32_t off[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) off[k] = ops[pc * kPer + k];
+        __syncthreads();  // the table's space becomes the operand buffers, the flag the two-part flag
+        if (twice) pieces = 0;
+        if (tid == 0) *two_part = 0;
+        if (pieces && live) {
+            for (int i0 = 0; i0 < n_loads; i0 += N) {
+                if (i0) load_pieces(i0);
+                char* dst = reinterpret_cast<char*>(mykeys + m0 * SD) + i0 * kpl * SD * 4;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    if (i0 + i >= n_loads) break;  // uniform
+                    const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if constexpr (KM == kKeyF32) {
+                            *reinterpret_cast<u32a*>(dst + off[k]) = w[k];
+                            low |= w[k] & 0xFFFFu;
+                        } else {
+                            *reinterpret_cast<u16a*>(dst + off[2 * k]) = (uint16_t)w[k];
+                            *reinterpret_cast<u16a*>(dst + off[2 * k + 1]) = (uint16_t)(w[k] >> 16);
+                        }
+                    }
+                    dst += kpl * SD * 4;
+                }
+            }
+            wave_sync_lds();
+        }
+    }
     if constexpr (KM == kKeyF32) __syncthreads();  // *two_part is cleared
-    if (live) {
-        const int E = nl * BDP;
+    if (live && !pieces) {
         int epad = BDP;
         while (epad < E && epad < 64) epad <<= 1;
         const int sub = lane / epad, kp = 64 / epad, trips = 32 / kp;
@@ -337,54 +433,58 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                     }
                 }
             };
-            if (trips >= 16)
-                for (int m0 = 0; m0 < trips; m0 += 16) take(m0, std::integral_constant<int, 16>{});
-            else if (trips == 8) take(0, std::integral_constant<int, 8>{});
+            if (trips >= 8)
+                for (int m0 = 0; m0 < trips; m0 += 8) take(m0, std::integral_constant<int, 8>{});
             else
                 for (int m0 = 0; m0 < trips; ++m0) take(m0, std::integral_constant<int, 1>{});
         }
         wave_sync_lds();
-        if (KM == kKeyF32 && met) {  // the key blocks' images under the block metric
-            low = 0;
-            for (int j = half; j < nl; j += 2) {
-                u32a* ks = mykeys + (j * kKeyRow + col) * SD;
-                uint32_t kw[SD];
-                float x[BDP];
-                lds_dwords<SD>(ks, kw);
-                slot_elems<BDP, KM>(kw, x);
-                const int blk = p.light[l0 + j];
-                to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, x);
+    }
+    if (KM == kKeyF32 && met && live) {  // the key blocks' images under the block metric
+        low = 0;
+        for (int j = half; j < nl; j += 2) {
+            u32a* ks = mykeys + (j * kKeyRow + col) * SD;
+            uint32_t kw[SD];
+            float x[BDP];
+            lds_dwords<SD>(ks, kw);
+            slot_elems<BDP, KM>(kw, x);
+            const int blk = p.light[l0 + j];
+            to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, x);
 #pragma unroll
-                for (int d = 0; d < BDP; ++d) {
-                    ks[d] = __float_as_uint(x[d]);
-                    low |= __float_as_uint(x[d]) & 0xFFFFu;
-                }
+            for (int d = 0; d < BDP; ++d) {
+                ks[d] = __float_as_uint(x[d]);
+                low |= __float_as_uint(x[d]) & 0xFFFFu;
             }
-            wave_sync_lds();
         }
+        wave_sync_lds();
     }
     // whether every key of the workgroup is exact in one bf16 part
     if (KM == kKeyF32 && low) *two_part = 1;
     __syncthreads();
-    const bool one_part = KM == kKeyBf16 || (KM == kKeyF32 && *two_part == 0);
+    const bool one_part = BDP == 2 || KM == kKeyBf16 || (KM == kKeyF32 && *two_part == 0);
     const float ex = one_part ? p.ex[0] : p.ex[1], es = one_part ? p.es[0] : p.es[1];
 
-    // A stage's codewords: four of the sixteen waves build stage it (they rotate), one codeword a
-    // thread; the rows load before the current stage's work and are written after it.
-    const int nst = WIDE ? (nc + kStageCw - 1) / kStageCw : 1;
+    // A stage's codewords, one per thread: with 1,024-codeword stages every wave builds, with smaller
+    // ones the waves take turns.  The rows load two stages ahead; the operand is written at the start
+    // of the stage before it, beside the other waves' work.  (A quarter codeword per thread, so that
+    // every wave builds 256-codeword stages too, took more instructions in all: 188 against 169 us.)
+    constexpr int kSc = stage_cw(BDP, WIDE), kTurns = kTileThreads / kSc;
+    const int nst = WIDE ? (nc + kSc - 1) / kSc : 1;
     const int n_it = nl * nst;
+    const int bcw = tid & (kSc - 1);
     float cw[BDP];
-    auto builds = [&](int it) { return it < n_it && (wave >> 2) == (it & 3); };
-    auto load_cw = [&](int it) {
-        const int j = WIDE ? it / nst : it;
-        const int st = WIDE ? it - j * nst : 0;
-        const int blk = p.light[l0 + j];
-        load_row<BDP>(cent + (int64_t)blk * nc * bd, min(st * kStageCw + (tid & 255), nc - 1), bd, p.vec, cw);
+    auto builds = [&](int it) { return it < n_it && wave / (kTileWaves / kTurns) == (it & (kTurns - 1)); };
+    int lj = 0, lst = 0;  // block and stage of the next load
+    auto load_next = [&](int it) {
+        if (builds(it)) {
+            const float* cb = cent + (int64_t)p.light[l0 + lj] * nc * bd;
+            load_row<BDP>(cb, min(lst * kSc + bcw, nc - 1), bd, p.vec, cw);
+        }
+        if (++lst == nst) { lst = 0; ++lj; }
     };
-    auto store_cw = [&](int it) {
-        const int j = WIDE ? it / nst : it;
-        const int st = WIDE ? it - j * nst : 0;
-        const int t = tid & 255;
+    // operand dword i of a codeword, from its row's first dword: [MFMA][half][row][4 dwords]
+    constexpr auto at_dw = [](int i) { return (i / 8) * 256 + ((i / 4) & 1) * 128 + (i & 3); };
+    auto store_cw = [&](int it, int j, int st) {
         if (met) {
             const int blk = p.light[l0 + j];
             to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, cw);
@@ -394,51 +494,88 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         uint32_t kd[8 * NM];
 #pragma unroll
         for (int i = 0; i < 8 * NM; ++i) kd[i] = 0;
-        const bool real = !WIDE || st * kStageCw + t < nc;
-        if (real) {
 #pragma unroll
-            for (int d = 0; d < BDP; d += 2) {
-                float v[2], h[2], m[2], l[2];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    v[u] = -2.0f * cw[d + u];
-                    h[u] = bf16_round(v[u]);
-                    v[u] -= h[u];
-                    m[u] = bf16_round(v[u]);
-                    l[u] = v[u] - m[u];
-                }
-                const uint32_t hw = pk_bf16(h[0], h[1]);
+        for (int d = 0; d < BDP; d += 2) {
+            float r0, r1, s0, s1;
+            const uint32_t hw = split2(-2.0f * cw[d], -2.0f * cw[d + 1], r0, r1);
+            const uint32_t mw = split2(r0, r1, s0, s1), lw = pk_bf16(s0, s1);
+            if constexpr (BDP == 2) {
+                kd[0] = kd[2] = kd[5] = hw;
+                kd[1] = kd[4] = mw;
+                kd[3] = lw;
+            } else {
                 kd[d / 2] = hw;
-                kd[(BDP + d) / 2] = pk_bf16(m[0], m[1]);
-                kd[(2 * BDP + d) / 2] = one_part ? pk_bf16(l[0], l[1]) : hw;
+                kd[(BDP + d) / 2] = mw;
+                kd[(2 * BDP + d) / 2] = one_part ? lw : hw;
             }
-            const float n1 = bf16_round(cn), r1 = cn - n1, n2 = bf16_round(r1), r2 = r1 - n2;
-            kd[3 * BDP / 2] = pk_bf16(n1, n2);
-            kd[3 * BDP / 2 + 1] = pk_bf16(r2, 1.0f);
-        } else {  // past the codebook's end: larger than any key's threshold
-            kd[3 * BDP / 2] = 0x7E80u;  // 2^126
+        }
+        float r1, u, r2;
+        split2(cn, 0.f, r1, u);
+        kd[kNorm] = split2(cn, r1, u, r2);
+        kd[kNorm + 1] = pk_bf16(r2, 1.0f);
+        if (WIDE && st * kSc + bcw >= nc) {  // past the codebook's end: 2^126, larger than any threshold
+#pragma unroll
+            for (int i = 0; i < 8 * NM; ++i) kd[i] = i == kNorm ? 0x7E80u : 0u;
         }
         // row of codeword w of its tile: a lane's 16 accumulators are then 16 consecutive codewords
-        const int w = t & 31;
+        const int w = bcw & 31;
         const int row = 8 * ((w >> 2) & 3) + 4 * (w >> 4) + (w & 3);
-        u32a* dst = ops + (it & 1) * Sh::kOps + (t >> 5) * NM * 256 + row * 4;
+        u32a* dst = ops + (it & 1) * Sh::kOps + (bcw >> 5) * NM * 256 + row * 4;
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                *reinterpret_cast<uint4*>(dst + m * 256 + h * 128) =
-                    make_uint4(kd[8 * m + 4 * h], kd[8 * m + 4 * h + 1], kd[8 * m + 4 * h + 2], kd[8 * m + 4 * h + 3]);
+        for (int i = 0; i < 8 * NM; i += 4)
+            *reinterpret_cast<uint4*>(dst + at_dw(i)) = make_uint4(kd[i], kd[i + 1], kd[i + 2], kd[i + 3]);
         if constexpr (!WIDE) {
-            u32a* rec = recs + (it & 1) * Sh::kRecs + (t >> 2) * Sh::kRec;
+            u32a* rec = recs + (it & 1) * Sh::kRecs + (bcw >> 2) * Sh::kRec;
 #pragma unroll
-            for (int d = 0; d < BDP; ++d) rec[(t & 3) * BDP + d] = __float_as_uint(cw[d]);
-            rec[4 * BDP + (t & 3)] = __float_as_uint(cn);
+            for (int d = 0; d < BDP; ++d) rec[(bcw & 3) * BDP + d] = __float_as_uint(cw[d]);
+            rec[4 * BDP + (bcw & 3)] = __float_as_uint(cn);
         }
     };
-    if (builds(0)) {
-        load_cw(0);
-        store_cw(0);
-    }
+    // every codeword of block j for key kk of the workgroup, over the lanes of a wave: the reference's
+    // chain, the first index of the smallest sqrt.  A wave busy with it holds the whole workgroup at
+    // the next barrier (it takes longer than a 256-codeword block), so the open pairs wait for the
+    // end, where the lanes share them, and this serves only those past the list's end.
+    auto scan_all = [&](int j, int kk) {
+        u32a* ks = keysL + (j * kKeyRow + kk) * SD;
+        uint32_t kwm[SD];
+        float xm[BDP];
+        lds_dwords<SD>(ks, kwm);
+        slot_elems<BDP, KM>(kwm, xm);
+        const float xmn = norm_p<BDP>(xm);
+#pragma unroll
+        for (int d = 0; d < BDP; ++d) xm[d] = -2.0f * xm[d];
+        const int blk = p.light[l0 + j];
+        const float* cb = cent + (int64_t)blk * nc * bd;
+        float be = INFINITY;  // the smallest clamped value, and the first index of its sqrt
+        uint32_t bn = 0x7FFFFFFFu;
+        constexpr int NB = BDP <= 4 ? 4 : BDP <= 8 ? 2 : 1;
+#pragma unroll 1
+        for (int n0 = lane; n0 < nc; n0 += 64 * NB) {
+            float c[NB][BDP];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) load_row<BDP>(cb, min(n0 + 64 * i, nc - 1), bd, p.vec, c[i]);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[i]);
+                // past the end: the last codeword again, which cannot win over itself
+                take_min(exact_e<BDP>(xm, xmn, c[i], norm_p<BDP>(c[i])), (uint32_t)min(n0 + 64 * i, nc - 1), be, bn);
+            }
+        }
+        if (bn == 0x7FFFFFFFu) bn = (uint32_t)lane;  // every value infinite
+        float bf = __builtin_sqrtf(be);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float of = __shfl_xor(bf, o);
+            const uint32_t on = (uint32_t)__shfl_xor((int)bn, o);
+            if (of < bf || (of == bf && on < bn)) { bf = of; bn = on; }
+        }
+        if (lane == 0) ks[0] = bn;
+        wave_sync_lds();
+    };
+
+    load_next(0);
+    if (builds(0)) store_cw(0, 0, 0);
+    load_next(1);
     __syncthreads();
 
     for (int j = 0, it = 0; j < nl; ++j) {
@@ -457,22 +594,32 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
             uint32_t kd[8 * NM];
 #pragma unroll
             for (int i = 0; i < 8 * NM; ++i) kd[i] = 0;
+            if constexpr (BDP == 2) {
+                if constexpr (KM == kKeyBf16) {
+                    kd[0] = kd[1] = kd[3] = kw[0];
+                } else {
+                    float r0, r1, t0, t1;
+                    kd[0] = kd[1] = kd[3] = split2(x[0], x[1], r0, r1);
+                    kd[2] = kd[4] = split2(r0, r1, t0, t1);
+                    kd[5] = pk_bf16(t0, t1);
+                }
+            } else
 #pragma unroll
             for (int d = 0; d < BDP; d += 2) {
                 uint32_t hw, third;
                 if constexpr (KM == kKeyBf16) {
                     hw = third = kw[d / 2];
                 } else {
-                    const float h0 = bf16_round(x[d]), h1 = bf16_round(x[d + 1]);
-                    hw = pk_bf16(h0, h1);
-                    third = one_part ? hw : pk_bf16(x[d] - h0, x[d + 1] - h1);
+                    float r0, r1;
+                    hw = split2(x[d], x[d + 1], r0, r1);
+                    third = one_part ? hw : pk_bf16(r0, r1);
                 }
                 kd[d / 2] = hw;
                 kd[(BDP + d) / 2] = hw;
                 kd[(2 * BDP + d) / 2] = third;
             }
-            kd[3 * BDP / 2] = 0x3F803F80u;
-            kd[3 * BDP / 2 + 1] = 0x3F80u | xu;
+            kd[kNorm] = 0x3F803F80u;
+            kd[kNorm + 1] = 0x3F80u | xu;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
                 uint4 v;
@@ -485,65 +632,92 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         }
         int m1 = 0x7FFFFFFF, m2 = 0x7FFFFFFF, mst = 0;
         for (int st = 0; st < nst; ++st, ++it) {
-            const bool bld = builds(it + 1);
-            if (bld) load_cw(it + 1);
+            if (builds(it + 1)) store_cw(it + 1, st + 1 == nst ? j + 1 : j, st + 1 == nst ? 0 : st + 1);
+            load_next(it + 2);
             if (live) {
+                // Tile t + 1's MFMA is issued before tile t's minima are taken, and its operand read
+                // a tile earlier still (the scheduling barriers keep that order).
                 const u32a* op = ops + (it & 1) * Sh::kOps + lane * 4;
+                auto opnd = [&](int t, int m) {
+                    return __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(op + (t * NM + m) * 256));
+                };
+                v8bf av[2][NM];
+                v16f acc[2];
+                auto issue = [&](int t) {
+                    v16f c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[t & 1][m], kb[m], c, 0, 0, 0);
+                    acc[t & 1] = c;
+                };
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    av[0][m] = opnd(0, m);
+                    av[1][m] = opnd(1, m);
+                }
+                issue(0);
                 int q1 = 0x7FFFFFFF, q2 = 0x7FFFFFFF;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < Sh::kTiles; ++t) {
+                    if (t + 2 < Sh::kTiles) {
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) {
-                        const uint4 w = *reinterpret_cast<const uint4*>(op + (t * NM + m) * 256);
-                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, w), kb[m], acc, 0, 0, 0);
+                        for (int m = 0; m < NM; ++m) av[t & 1][m] = opnd(t + 2, m);
                     }
+                    if (t + 1 < Sh::kTiles) issue(t + 1);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {  // codewords 32 t + 16 half + 8 u ... + 7
-                        int b[8];
+                    for (int u = 0; u < 16 / kGc; ++u) {  // codewords 32 t + 16 half + kGc u ... + kGc - 1
+                        int b[kGc];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) b[i] = __float_as_int(acc[8 * u + i]);
-                        int v = min(min(b[0], b[1]), b[2]);
-                        v = min(min(v, b[3]), b[4]);
-                        v = min(min(v, b[5]), b[6]);
-                        v = min(v, b[7]);
-                        v = (v & -16) | (2 * t + u);
+                        for (int i = 0; i < kGc; ++i) b[i] = __float_as_int(acc[t & 1][kGc * u + i]);
+                        int v = min(min(b[0], b[1]), b[2]);  // v_min3_i32
+#pragma unroll
+                        for (int i = 3; i + 1 < kGc; i += 2) v = min(min(v, b[i]), b[i + 1]);
+                        v = min(v, b[kGc - 1]);
+                        v = (v & -16) | ((16 / kGc) * (t % kTagTiles) + u);
                         q2 = med3_s(q1, q2, v);
                         q1 = min(q1, v);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (WIDE) {
+                        if (t % kTagTiles == kTagTiles - 1) {
+                            m2 = min(min(max(m1, q1), m2), q2);
+                            mst = q1 < m1 ? st * (Sh::kTiles / kTagTiles) + t / kTagTiles : mst;
+                            m1 = min(m1, q1);
+                            q1 = q2 = 0x7FFFFFFF;
+                        }
+                    }
                 }
-                if constexpr (WIDE) {
-                    m2 = min(min(max(m1, q1), m2), q2);
-                    mst = q1 < m1 ? st : mst;
-                    m1 = min(m1, q1);
-                } else {
+                if constexpr (!WIDE) {
                     m1 = q1;
                     m2 = q2;
                 }
             }
             if (live && (!WIDE || st + 1 == nst)) {
                 // threshold from the key's minimum (its tag in the low bits), and whether one group
-                // alone reaches it (past 256 codewords: one group per lane)
+                // alone reaches it.  Bit l of the masks below is key l; a key's other lane is 32 bits up.
                 int pa, pb;
                 pair32((m1 & -32) | ((m1 & 15) << 1) | half, pa, pb);
                 const int pk = min(pa, pb);
                 const float mt = fmaxf(__int_as_float(pk & -32), 0.f) * (1.0f + 0x1.0p-17f);
                 const float thr = mt + es * fmaxf(mt - dlt, 0.f) + ex * xn + 0x1.0p-100f;
-                const bool c1 = __int_as_float(m1 & -32) <= thr, c2 = __int_as_float(m2 & -32) <= thr;
-                int fa, fb;
-                pair32((c1 ? 1 : 0) + (c2 ? 4 : 0), fa, fb);
-                bool open = !(xn < 0x1.0p120f) || bad[j] != 0 || (WIDE ? fa + fb >= 4 : fa + fb != 1);
+                const uint64_t b1 = __builtin_amdgcn_ballot_w64(__int_as_float(m1 & -32) <= thr);
+                const uint64_t b2 = __builtin_amdgcn_ballot_w64(__int_as_float(m2 & -32) <= thr);
+                const uint64_t fin = __builtin_amdgcn_ballot_w64(xn < 0x1.0p120f);
+                uint32_t ok = (uint32_t)fin & (uint32_t)(b1 ^ (b1 >> 32)) & ~(uint32_t)(b2 | (b2 >> 32));
+                if (__builtin_amdgcn_readfirstlane(bad[j])) ok = 0;
                 float m2x[BDP];
 #pragma unroll
                 for (int d = 0; d < BDP; ++d) m2x[d] = -2.0f * x[d];
-                // the reference's arithmetic inside the group: this lane's half of it, or (past 256
-                // codewords) its own group
-                constexpr int NC = WIDE ? 8 : 4;
-                const int tag = WIDE ? m1 & 15 : (pk >> 1) & 15;
-                const int first = WIDE ? mst * kStageCw + (tag >> 1) * 32 + half * 16 + (tag & 1) * 8
-                                       : (tag >> 1) * 32 + (pk & 1) * 16 + (tag & 1) * 8 + half * 4;
+                // the reference's arithmetic inside the group: half of its codewords on each of the key's lanes
+                constexpr int NC = kGc / 2;
+                const int tag = (pk >> 1) & 15;
+                int first = (WIDE ? tag * 32 : (tag >> 1) * 32 + (tag & 1) * 8) + (pk & 1) * 16 + half * NC;
                 Top2 best[NC];
                 if constexpr (WIDE) {
+                    int sa, sb;
+                    pair32(m1, pa, pb);
+                    pair32(mst, sa, sb);
+                    first += (pa < pb ? sa : sb) * (32 * kTagTiles);
                     const int blk = p.light[l0 + j];
                     const float* cb = cent + (int64_t)blk * nc * bd;
                     float c[NC][BDP];
@@ -553,7 +727,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                     for (int i = 0; i < NC; ++i) {
                         if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[i]);
                         const float e = exact_e<BDP>(m2x, xn, c[i], norm_p<BDP>(c[i]));
-                        best[i] = {first + i < nc ? __float_as_int(e) : kInfBits, kInfBits, first + i};
+                        best[i] = {first + i < nc ? __float_as_int(e) : kInfBits, kInfBits, i};
                     }
                 } else {
                     uint32_t rec[Sh::kRec];
@@ -564,79 +738,87 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
 #pragma unroll
                         for (int d = 0; d < BDP; ++d) c[d] = __uint_as_float(rec[i * BDP + d]);
                         const float e = exact_e<BDP>(m2x, xn, c, __uint_as_float(rec[4 * BDP + i]));
-                        best[i] = {__float_as_int(e), kInfBits, first + i};
+                        best[i] = {__float_as_int(e), kInfBits, i};
                     }
                 }
 #pragma unroll
                 for (int w = 1; w < NC; w <<= 1)
 #pragma unroll
                     for (int i = 0; i < NC; i += 2 * w) best[i] = join(best[i], best[i + w]);
-                int ea, eb, na, nb2, ga, gb;
+                int ea, eb;
                 pair32(best[0].e1, ea, eb);
-                pair32(best[0].e2, ga, gb);
-                pair32(best[0].n, na, nb2);
-                int code = ea < eb ? na : nb2;
-                const float e1 = __int_as_float(min(ea, eb));
-                const float e2 = __int_as_float(min(min(ga, gb), max(ea, eb)));
+                const int e1 = min(ea, eb);
+                const bool mine = best[0].e1 == e1;
+                const float e2 = __int_as_float(mine ? best[0].e2 : best[0].e1);
+                const uint64_t bm = __builtin_amdgcn_ballot_w64(mine);
                 // below t the smaller value's correctly rounded sqrt is the smaller one
-                open = open || !(e1 < e2 * 0x1.ffffep-1f - 0x1.0p-146f);
-                uint64_t todo = __builtin_amdgcn_ballot_w64(open) & 0xFFFFFFFFull;
-#pragma unroll 1
-                while (todo) {  // rare: every codeword of the block for key m, over the wave's lanes
-                    const int m = __builtin_ctzll(todo);
-                    todo &= todo - 1;
-                    uint32_t kwm[SD];
-                    float xm[BDP];
-                    lds_dwords<SD>(mykeys + (j * kKeyRow + m) * SD, kwm);
-                    slot_elems<BDP, KM>(kwm, xm);
-                    const float xmn = norm_p<BDP>(xm);
-#pragma unroll
-                    for (int d = 0; d < BDP; ++d) xm[d] = -2.0f * xm[d];
-                    float bf = INFINITY;
-                    int bn = 0x7FFFFFFF;
-                    if constexpr (WIDE) {
-                        const int blk = p.light[l0 + j];
-                        const float* cb = cent + (int64_t)blk * nc * bd;
-#pragma unroll 1
-                        for (int n0 = lane; n0 < nc; n0 += 256) {
-                            float c[4][BDP];
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) load_row<BDP>(cb, min(n0 + 64 * i, nc - 1), bd, p.vec, c[i]);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                const int n = n0 + 64 * i;
-                                if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[i]);
-                                const float f = __builtin_sqrtf(exact_e<BDP>(xm, xmn, c[i], norm_p<BDP>(c[i])));
-                                if (n < nc && (f < bf || (f == bf && n < bn))) { bf = f; bn = n; }
-                            }
-                        }
-                    } else {
-                        uint32_t rec[Sh::kRec];
-                        lds_dwords<Sh::kRec>(recs + (it & 1) * Sh::kRecs + lane * Sh::kRec, rec);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            float c[BDP];
-#pragma unroll
-                            for (int d = 0; d < BDP; ++d) c[d] = __uint_as_float(rec[i * BDP + d]);
-                            const float f = __builtin_sqrtf(exact_e<BDP>(xm, xmn, c, __uint_as_float(rec[4 * BDP + i])));
-                            if (f < bf || (f == bf && 4 * lane + i < bn)) { bf = f; bn = 4 * lane + i; }
-                        }
-                    }
-#pragma unroll
-                    for (int o = 32; o > 0; o >>= 1) {
-                        const float of = __shfl_xor(bf, o);
-                        const int on = __shfl_xor(bn, o);
-                        if (of < bf || (of == bf && on < bn)) { bf = of; bn = on; }
-                    }
-                    if (col == m) code = bn;
-                }
+                const uint64_t far = __builtin_amdgcn_ballot_w64(__int_as_float(e1) < e2 * 0x1.ffffep-1f - 0x1.0p-146f);
+                ok &= (uint32_t)(far & (far >> 32)) & (uint32_t)(bm ^ (bm >> 32));
                 // the code takes the place of the block's key elements
-                if (half == 0) ks[0] = (uint32_t)code;
+                if (mine && ((ok >> col) & 1)) ks[0] = (uint32_t)(first + best[0].n);
+                const uint32_t todo = ~ok;
+                if (todo) {  // rare: to the list for the end; what does not fit there is scanned here
+                    int at = 0;
+                    if (lane == 0) at = (int)atomicAdd(n_open, (uint32_t)__popc(todo));
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    const int pos = at + __popc(todo & ((1u << col) - 1u));
+                    if (half == 0 && ((todo >> col) & 1) && pos < kOpenCap)
+                        open_list[pos] = (uint16_t)(j * kTileKeys + wave * 32 + col);
+                    if (at + __popc(todo) > kOpenCap) {
+                        wave_sync_lds();
+                        for (uint32_t t = todo; t; t &= t - 1)
+                            if (at++ >= kOpenCap) scan_all(j, wave * 32 + __builtin_ctz(t));
+                    }
+                }
                 wave_sync_lds();
             }
-            if (bld) store_cw(it + 1);
             __syncthreads();
         }
+    }
+    // The pairs put off, published by the loop's last barrier: 16 lanes per 256 codewords of a pair,
+    // 16 codewords a lane; (sqrt bits, index) pairs meet in a 64-bit LDS minimum, which orders them as
+    // the reference does (the operand buffers' space).
+    const int n_put = nl > 0 ? min((int)__builtin_amdgcn_readfirstlane(*n_open), kOpenCap) : 0;
+    if (n_put) {
+        unsigned long long* res = reinterpret_cast<unsigned long long*>(tile_lds);
+        if (tid < n_put) res[tid] = ~0ull;
+        __syncthreads();
+        const int parts = (nc + 255) / 256;
+        for (int i = tid >> 4; i < n_put * parts; i += kTileThreads / 16) {
+            const int en = i / parts, n1 = (i - en * parts) * 256 + (tid & 15);
+            const int j = open_list[en] / kTileKeys;
+            uint32_t kwm[SD];
+            float xm[BDP];
+            lds_dwords<SD>(keysL + (j * kKeyRow + open_list[en] % kTileKeys) * SD, kwm);
+            slot_elems<BDP, KM>(kwm, xm);
+            const float xmn = norm_p<BDP>(xm);
+#pragma unroll
+            for (int d = 0; d < BDP; ++d) xm[d] = -2.0f * xm[d];
+            const int blk = p.light[l0 + j];
+            const float* cb = cent + (int64_t)blk * nc * bd;
+            float be = INFINITY;
+            uint32_t bn = 0x7FFFFFFFu;
+            constexpr int NB = BDP <= 4 ? 16 : BDP <= 8 ? 4 : 1;
+#pragma unroll 1
+            for (int n0 = n1; n0 < n1 + 256; n0 += 16 * NB) {
+                float c[NB][BDP];
+#pragma unroll
+                for (int u = 0; u < NB; ++u) load_row<BDP>(cb, min(n0 + 16 * u, nc - 1), bd, p.vec, c[u]);
+#pragma unroll
+                for (int u = 0; u < NB; ++u) {
+                    if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[u]);
+                    take_min(exact_e<BDP>(xm, xmn, c[u], norm_p<BDP>(c[u])), (uint32_t)min(n0 + 16 * u, nc - 1), be, bn);
+                }
+            }
+            if (bn == 0x7FFFFFFFu) bn = (uint32_t)min(n1, nc - 1);  // every value infinite
+            atomicMin(&res[en], ((unsigned long long)__float_as_uint(__builtin_sqrtf(be)) << 32) | bn);
+        }
+        __syncthreads();
+        if (tid < n_put) {
+            const int j = open_list[tid] / kTileKeys;
+            keysL[(j * kKeyRow + open_list[tid] % kTileKeys) * SD] = (uint32_t)res[tid];
+        }
+        __syncthreads();
     }
     if (!live) return;
 
@@ -700,15 +882,15 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     const ssq_encode_args& a = tp.a;
     constexpr bool raw16 = KM != kKeyF32;
     int nbc = tp.n_light > 0 ? tp.n_light : 1;
-    while (nbc > 1 && tile_smem<BDP>(nbc, raw16, WIDE) > kTileSmemCap) --nbc;
+    while (nbc > 1 && tile_smem<BDP, WIDE>(nbc, raw16) > kTileSmemCap) --nbc;
     tp.fold = ssq_encode_fold(&a, kTileKeys);
     const int64_t n_keys = tp.fold ? (int64_t)a.batch * a.seq_len : a.seq_len;
     const int64_t xg = (n_keys + kTileKeys - 1) / kTileKeys;
     const int64_t groups = xg * (tp.fold ? a.num_kv_heads : (int64_t)a.batch * a.num_kv_heads);
     // Smaller chunks of blocks until the workgroups fill the chip: a few keys (a decode step's
     // append) take one block per workgroup.  Past 256 codewords a block is long, so the chunks
-    // shrink until about four workgroups per CU even out the last round.
-    const int64_t want_wg = (WIDE ? 4 : 1) * (int64_t)ssq_device_cus();
+    // shrink until there are two workgroups per CU to even out the last round.
+    const int64_t want_wg = (WIDE ? 2 : 1) * (int64_t)ssq_device_cus();
     if (tp.n_light > 0) {
         int chunks = (tp.n_light + nbc - 1) / nbc;
         if (groups * chunks < want_wg) {
@@ -719,6 +901,16 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     }
     tp.nbc = nbc;
     tp.chunks = tp.n_light > 0 ? (tp.n_light + nbc - 1) / nbc : 1;
+    // whole key rows in 16-byte pieces: chunks that use most of a row, aligned rows in the staged
+    // type, pieces that divide a wave
+    const int elem = raw16 ? 2 : 4;
+    const int pieces = a.head_dim * elem / 16;
+    const bool staged_type = raw16 || a.k_dtype == SSQ_F32;
+    tp.pieces = BDP < 16 && 2 * nbc * BDP > a.head_dim && a.block_dim == BDP && staged_type && (a.head_dim * elem) % 16 == 0 && pieces >= 2 && pieces <= 64 &&
+                        (pieces & (pieces - 1)) == 0 && (uintptr_t)a.keys % 16 == 0 && (a.k_sb * elem) % 16 == 0 &&
+                        (a.k_sh * elem) % 16 == 0 && (a.k_ss * elem) % 16 == 0
+                    ? pieces
+                    : 0;
     const int cw = ssq_code_width(a.n_centroids);
     tp.row_codes = tp.chunks == 1 && (a.n_blocks * cw) % 16 == 0 && (uintptr_t)a.codes % 16 == 0 &&
                    (a.c_sb * cw) % 16 == 0 && (a.c_sh * cw) % 16 == 0 && (a.c_st * cw) % 16 == 0;
@@ -726,7 +918,7 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     SSQ_UNSUPPORTED(groups <= 0x7fffffff && wgs <= 0x7fffffff, "too many keys for one encode launch");
     tp.xg = (int)xg;
     tp.groups = (int)groups;
-    const size_t smem = tile_smem<BDP>(nbc, raw16, WIDE);
+    const size_t smem = tile_smem<BDP, WIDE>(nbc, raw16);
     SSQ_UNSUPPORTED(smem <= kTileSmemCap, "block too large for the MFMA encode");
     const int rc = ssq_allow_lds((const void*)k_encode_tile<BDP, KM, WIDE>, (int)kTileSmemCap,
                                  "hipFuncSetAttribute(encode tile)");
@@ -752,7 +944,9 @@ int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st) {
     const int bd = a->block_dim;
     for (int two = 0; two < 2; ++two) {  // the bound of the file comment, rounded up
         const double gr = 1.001 * (bd + 2) * 0x1.0p-23;
-        const double A = 1.02 * (3 * bd + 4) * 0x1.0p-23 + bd * 0x1.0p-24 + (two ? 1.53 * 0x1.0p-18 : 0.0);
+        const int terms = (bd <= 2 ? 6 : 3) * bd + 4;
+        const double left = bd <= 2 ? 0x1.0p-24 : two ? 1.53 * 0x1.0p-18 : 0.0;
+        const double A = 1.02 * terms * 0x1.0p-23 + bd * 0x1.0p-24 + left;
         const double B = A + gr;
         tp.ex[two] = (float)(12.6 * B * 1.001);
         tp.es[two] = (float)((0x1.0p-20 + 6.2 * B) * 1.001);
@@ -763,7 +957,7 @@ int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st) {
     }
     const int64_t al = bd == 2 ? 8 : 16;
     tp.vec = (bd == 2 || bd == 4 || bd == 8 || bd == 16) && (uintptr_t)a->cent % al == 0 && (a->cent_sh * 4) % al == 0;
-    const bool wide = a->n_centroids > kStageCw;
+    const bool wide = a->n_centroids > 256;
     const int bdp = bd <= 2 ? 2 : bd <= 4 ? 4 : bd <= 8 ? 8 : 16;
     switch (bdp * 2 + (wide ? 1 : 0)) {
         case 4: return launch_tile_keys<2, false>(tp, st);

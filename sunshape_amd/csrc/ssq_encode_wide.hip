@@ -38,32 +38,6 @@ __device__ __forceinline__ float stage_dist(const float* x, float xn, const floa
     return MM ? mm_dist2(x, xn, c, cn[j], w) : direct_dist2(x, c, w);
 }
 
-// A codeword's pre-sqrt value v, clamped as the reference's sqrt(clamp_min(., 0)) clamps it (NaN
-// and negatives: 0), against the smallest clamped value so far, e_min >= 0.  The common test,
-// !(v >= e_min), holds whenever the clamped value is below e_min (v < e_min, or v NaN, or v <= 0
-// while e_min > 0); the clamp and the exact test follow only then.  New minima are rare after a
-// lane's first codewords, and the empty volatile asm statements keep these branches, so that
-// nothing past the common test is evaluated for every codeword.  The index moves when the new
-// value's correctly rounded sqrt is below e_min's.  A correctly rounded sqrt merges
-// pre-sqrt values less than 2^-21 apart relatively at most (below 2^-126, a few units of the
-// smallest subnormal), so a value below t = e_min (1 - 2^-20) - 2^-146 has the smaller sqrt;
-// between t and e_min the two sqrts are compared.
-__device__ __forceinline__ void take_min(float v, uint32_t j, float& e_min, uint32_t& j_best) {
-    if (!(v >= e_min)) {
-        __asm__ volatile("");
-        const float vc = v > 0.f ? v : 0.f;
-        if (!(vc < e_min)) return;
-        const float t = e_min * 0x1.ffffep-1f - 0x1.0p-146f;
-        if (vc < t) {
-            j_best = j;
-        } else {
-            __asm__ volatile("");
-            if (__builtin_sqrtf(vc) < __builtin_sqrtf(e_min)) j_best = j;
-        }
-        e_min = vc;
-    }
-}
-
 // one LDS stage's codewords sl, sl + S, ... < n (ONE: S == 1) in ascending order; with the block
 // dim known, eight codewords' distances are computed before their minimum checks, so that their
 // LDS reads are in flight together
