@@ -7,6 +7,9 @@ int ssq_launch_merge(const ssq_decode_args& a, int n_splits, const float* ws_o, 
 // the 4x4-MFMA-scores kernel (ssq_decode_paged_q4.hip)
 bool ssq_decode_q4_shape(const ssq_decode_args* a);
 size_t ssq_decode_q4_smem(const ssq_decode_args* a, int rg, int split_len);
+size_t ssq_decode_q4_cut_smem(const ssq_decode_args* a, int rg, int pages);
+bool ssq_decode_q4_has_cut(const ssq_decode_args* a, int rows);
+int ssq_decode_q4_merge_cut(const SsqPagedParams& mp, hipStream_t st);
 int ssq_decode_q4_launch(const SsqPagedParams& mp, const dim3& grid, hipStream_t st);
 
 namespace {
@@ -42,6 +45,38 @@ void pt_dims(const ssq_decode_args& a, SsqPagedParams& mp) {
                 ((uintptr_t)a.pt + 2 * (uintptr_t)mp.hoff[0]) % 16 == 0 && (a.pt_sb * 2) % 16 == 0 &&
                 (a.pt_sh * 2) % 16 == 0 && (a.pt_st * 2) % 16 == 0;
     for (int i = 1; i < mp.n_hd; ++i) mp.pt_vec = mp.pt_vec && mp.hoff[i] == mp.hoff[0] + i;
+}
+
+// Length-balanced pages (SsqCut) where a batch has at least as many (sequence, KV head) pairs as the
+// device has CUs (fewer pairs run splits of the longest length, one round of them, which measured
+// faster there: 16 x 8 pairs of 4,096 tokens, 42 against 47 us), on the 4x4-MFMA kernel, one workgroup
+// per CU with at least a tile per wave.  The codebook is staged once per workgroup, and a segment's
+// last reloads are the next segment's first tiles.  kCutSeqBytes: what a CU streams during a
+// segment's prologue and merge (about 4 us at 27 KB/us).  Per call, one workgroup per pair against
+// this, 32/8 heads, head_dim 128, 64 blocks of dim 2: 48 sequences of log-spread lengths up to 8,192, 81 ->
+// 41 us; 64 up to 16,384, 168 -> 79 us; 48 of 8,192 each, 204 -> 177 us; 64 of 4,096 each, 126 -> 123 us.
+constexpr int kCutSeqBytes = 110 * 1000;
+void plan_cut(const ssq_decode_args& a, int rows, bool pt_vec, SsqMfmaPlan& pl) {
+    pl.cut_wg = 0;
+    if (!pl.q4 || pl.ct || pl.n_groups != 1 || a.num_splits != 0) return;
+    if ((int64_t)a.batch * a.num_kv_heads < ssq_device_cus()) return;
+    if (!ssq_decode_q4_has_cut(&a, rows) || (a.heavy_mask[0] && !pt_vec)) return;
+    const int n_wg = ssq_device_cus() / a.num_kv_heads;
+    if (n_wg < 1) return;
+    const int token_bytes = a.code_bits == 4 || a.code_bits == 6 ? a.n_blocks / 2 : a.n_blocks;
+    const int seq = (kCutSeqBytes / (token_bytes + 2 * a.value_dim) + 63) & ~63;
+    const int64_t cost = (int64_t)a.batch * (a.seq_len + seq);
+    if (cost + (int64_t)n_wg * 1024 > 0x7fffffff) return;
+    const int least = 8 * kTileTok;
+    int64_t most = (cost + n_wg - 1) / n_wg > least ? (cost + n_wg - 1) / n_wg : least;  // tokens of a segment
+    if (most > a.seq_len) most = a.seq_len;
+    const int pages = (int)(most / kPage) + 8;
+    if (ssq_decode_q4_cut_smem(&a, pl.rg, pages) > kMaxSmem) return;
+    pl.cut_wg = n_wg;
+    pl.cut_min = least;
+    pl.cut_seq = seq;
+    pl.cut_pages = pages;
+    pl.ws_bytes = (size_t)n_wg * a.num_kv_heads * 2 * rows * (a.value_dim + 2) * 4;
 }
 
 bool plan(const ssq_decode_args* a, SsqMfmaPlan& pl) {
@@ -159,6 +194,7 @@ bool plan(const ssq_decode_args* a, SsqMfmaPlan& pl) {
     if (pl.smem > kMaxSmem) return false;
     const size_t n_rows_all = (size_t)a->batch * a->num_q_heads * a->q_len;
     pl.ws_bytes = !nv && pl.n_splits > 1 ? (size_t)pl.n_splits * n_rows_all * (a->value_dim + 2) * 4 : 0;
+    plan_cut(*a, rows, dims.pt_vec != 0, pl);
     return true;
 }
 
@@ -198,6 +234,17 @@ int ssq_decode_mfma(const ssq_decode_args* a, void* workspace, size_t ws_bytes, 
     mp.ws_m = ws ? ws + (size_t)pl.n_splits * n_rows_all * a->value_dim : nullptr;
     mp.ws_l = ws ? mp.ws_m + (size_t)pl.n_splits * n_rows_all : nullptr;
     int rc;
+    if (pl.q4 && pl.cut_wg) {
+        mp.cut_wg = pl.cut_wg;
+        mp.cut_min = pl.cut_min;
+        mp.cut_seq = pl.cut_seq;
+        mp.cut_pages = pl.cut_pages;
+        const size_t part_rows = (size_t)pl.cut_wg * a->num_kv_heads * 2 * mp.rows;
+        mp.ws_m = ws + part_rows * a->value_dim;
+        mp.ws_l = mp.ws_m + part_rows;
+        rc = ssq_decode_q4_launch(mp, dim3(pl.cut_wg * a->num_kv_heads, 1, 1), st);
+        return rc ? rc : ssq_decode_q4_merge_cut(mp, st);
+    }
     if (pl.q4) {
         rc = ssq_decode_q4_launch(mp, dim3(mp.a.batch * mp.a.num_kv_heads, pl.n_splits, pl.n_groups), st);
         if (rc) return rc;

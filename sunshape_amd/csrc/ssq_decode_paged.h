@@ -19,6 +19,84 @@ struct SsqPagedParams {
     float* ws_o;
     float* ws_m;
     float* ws_l;
+    // length-balanced pages (SsqCut): workgroups per KV head (0: one per (sequence, split)), the
+    // smallest share of a workgroup and a sequence's fixed cost, both in tokens; the LDS page slots
+    int cut_wg, cut_min, cut_seq, cut_pages;
+};
+
+// Length-balanced work of the paged 4x4-MFMA kernel.  The host cannot see seq_lens, and a plan for the
+// longest possible sequence leaves a batch of mixed lengths waiting for the longest one.  So the
+// sequences of a KV head are laid end to end on a cost axis, cut_seq + len tokens each (the fixed part
+// is a segment's prologue and merge), and cut_wg workgroups take equal shares [w * share, (w + 1) *
+// share) of it.  A sequence inside one share is written out by its workgroup; one that spans several
+// leaves partials, slot 0 of a workgroup for the sequence its share starts in and slot 1 for a later
+// one that it does not finish, which k_merge_cut combines.  Every number here is a function of
+// seq_lens alone, so the decode workgroups and the merge agree without exchanging anything.
+struct SsqCut {
+    int share, total;
+    int c0, v0;  // this lane's cost and inclusive sum over the first 64 sequences
+    __device__ __forceinline__ static int len(const ssq_decode_args& a, int b) {
+        return max(0, min(a.seq_lens[b], a.seq_len));
+    }
+    // token position of cost position x of a sequence of L tokens: whole 64-token tiles
+    __device__ __forceinline__ static int token(int x, int fixed, int L) {
+        x -= fixed;
+        return x <= 0 ? 0 : x >= L ? L : x & ~63;
+    }
+    // inclusive wave sum: row shifts by 1, 2, 4 and 8, then lane 15 and lane 31 of the rows below
+    __device__ __forceinline__ static int scan(int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+        return v;
+    }
+    __device__ __forceinline__ static int cost(const ssq_decode_args& a, int b, int fixed) {
+        return b < a.batch ? len(a, b) + fixed : 0;
+    }
+    // (the whole wave calls this and the two below)
+    __device__ __forceinline__ void init(const ssq_decode_args& a, int lane, int n_wg, int fixed, int least) {
+        c0 = cost(a, lane, fixed);
+        v0 = scan(c0);
+        total = __builtin_amdgcn_readlane(v0, 63);
+        for (int b = SSQ_WAVE; b < a.batch; b += SSQ_WAVE)
+            total += __builtin_amdgcn_readlane(scan(cost(a, b + lane, fixed)), 63);
+        share = (max((total + n_wg - 1) / n_wg, least) + 63) & ~63;
+    }
+    // the sequence that holds cost position x < total, and its start
+    __device__ __forceinline__ void find(const ssq_decode_args& a, int lane, int x, int fixed, int& b, int& s) const {
+        int base = 0, c = c0, v = v0;
+        for (int f = 0;;) {
+            const uint64_t hit = __builtin_amdgcn_ballot_w64(base + v > x);
+            if (hit) {
+                const int l = __builtin_ctzll(hit);
+                b = f + l;
+                s = base + __builtin_amdgcn_readlane(v - c, l);
+                return;
+            }
+            base += __builtin_amdgcn_readlane(v, 63);
+            f += SSQ_WAVE;
+            if (f >= a.batch) break;  // not reached for x < total
+            c = cost(a, f + lane, fixed);
+            v = scan(c);
+        }
+        b = a.batch - 1;
+        s = x;
+    }
+    // sequence b's start and length
+    __device__ __forceinline__ void locate(const ssq_decode_args& a, int lane, int b, int fixed, int& s, int& L) const {
+        int base = 0, c = c0, v = v0;
+        for (int f = 0; b >= f + SSQ_WAVE;) {
+            base += __builtin_amdgcn_readlane(v, 63);
+            f += SSQ_WAVE;
+            c = cost(a, f + lane, fixed);
+            v = scan(c);
+        }
+        s = base + __builtin_amdgcn_readlane(v - c, b & 63);
+        L = __builtin_amdgcn_readlane(c, b & 63) - fixed;
+    }
 };
 
 namespace {

@@ -66,6 +66,14 @@ inline size_t q4_smem(const ssq_decode_args& a, int RP, int split_len, int W) {
     return main > merge ? main : merge;
 }
 
+// Length-balanced pages: the codebook stays for all of a workgroup's segments, so the waves' merge has
+// its own space: codebook | strips | merge [waves][RP][Dv + 2] | pages [2][cut_pages] |
+// first tiles' pages [waves][4]
+inline size_t q4_cut_smem(const ssq_decode_args& a, int RP, int pages, int W) {
+    return (size_t)q4_cb_floats(a.head_dim, a.n_centroids) * 4 + q4_strip_bytes(RP, W) +
+           (size_t)W * RP * (a.value_dim + 2) * 4 + 2 * (size_t)pages * 4 + (size_t)W * 16;
+}
+
 // The halves of issue_tile (ssq_decode_paged.h), for the one-register-set pipeline: a tile's codes
 // are reloaded as soon as its scores are done, its values as soon as its P.V is done.
 template <int NB, int DT, int PB>
@@ -397,7 +405,8 @@ __device__ __forceinline__ void tile_extra_scores(const MfmaParams& p, const flo
 // never allows.
 // MK: an additive mask; HV: passthrough blocks (1: 8 or 16 consecutive 16-bit values per token, 2:
 // any layout and dtype); both with byte codes only.
-template <int KD, int BD, int R4, int DT, int VT, int PB, int W, bool CT, bool MK, int HV>
+// CUT: length-balanced pages (SsqCut), a build of its own: its loop over segments costs scalar registers.
+template <int KD, int BD, int R4, int DT, int VT, int PB, int W, bool CT, bool MK, int HV, bool CUT>
 __global__ __launch_bounds__(W * SSQ_WAVE) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
 void k_decode_paged_q4(const MfmaParams p) {
     static_assert(!CT || (W == 8 && DT == 8), "contiguous rows: 8 waves, 128-dim values");
@@ -412,21 +421,58 @@ void k_decode_paged_q4(const MfmaParams p) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr bool cut = CUT;
+    static_assert(!CUT || (W == 8 && !CT && !MK), "length-balanced pages: 8 waves, no mask");
     const int bk = blockIdx.x;
     const int split = blockIdx.y;
-    const int b = bk / a.num_kv_heads;
-    const int kv = bk - b * a.num_kv_heads;
+    int b = cut ? 0 : bk / a.num_kv_heads;
+    const int kv = cut ? bk % a.num_kv_heads : bk - b * a.num_kv_heads;
     const int nc = a.n_centroids;
     const int row0 = blockIdx.z * p.rg;       // this workgroup's query rows: row0 .. row0 + nr - 1
     const int nr = min(p.rg, p.rows - row0);  // <= RP
-    const int T = CT ? a.seq_len : min(a.seq_lens[b], a.seq_len);
-    const int t_begin = split * p.split_len;
-    const int t_end = min(T, t_begin + p.split_len);
 
     float* cb = smem;
     uint8_t* strips = reinterpret_cast<uint8_t*>(smem + q4_cb_floats(KD, nc));
     uint16_t* pstrip = reinterpret_cast<uint16_t*>(strips) + wave * RP * kTileTok;
-    int* pages = reinterpret_cast<int*>(strips + (size_t)kWaves * RP * kTileTok * 2);  // paged only
+    float* mspace = cut ? reinterpret_cast<float*>(strips + (size_t)kWaves * RP * kTileTok * 2) : smem;
+    int* pages = cut ? reinterpret_cast<int*>(mspace + kWaves * RP * (DT * 16 + 2))
+                     : reinterpret_cast<int*>(strips + (size_t)kWaves * RP * kTileTok * 2);  // paged only
+    int* const pages0 = pages;                  // (length-balanced: two slices of cut_pages slots, in turn,
+    int* first_pg = pages0 + 2 * p.cut_pages;  // and [waves][4] slots)
+
+    // the codebook goes global -> LDS directly: 1 KiB chunks, lane l's 16 bytes at chunk + 16 l;
+    // the tail chunk's lanes past the end re-read the last float4 into the padding
+    auto stage_codebook = [&]() {
+        const float* cent = a.cent + (int64_t)kv * a.cent_sh;
+        const int n4 = KD * nc / 4;
+        const int n_chunks = (n4 + 63) / 64;
+        for (int c = wave; c < n_chunks; c += kWaves) {
+            const int i = min(c * 64 + lane, n4 - 1);
+            __builtin_amdgcn_global_load_lds(cent + 4 * i, (__attribute__((address_space(3))) void*)(cb + 256 * c), 16,
+                                             0, 0);
+        }
+    };
+
+    // Length-balanced pages: this workgroup's share [lo, hi) of the cost axis, the sequence at hand and
+    // its start on the axis.
+    SsqCut ct{0, 0, 0, 0};
+    int lo = 0, hi = 0, s_at = 0;
+    if (cut) {
+        stage_codebook();
+        ct.init(a, lane, p.cut_wg, p.cut_seq, p.cut_min);
+        lo = (bk / a.num_kv_heads) * ct.share;
+        hi = lo + ct.share;
+        if (lo >= ct.total) {  // uniform over the workgroup
+            __builtin_amdgcn_s_waitcnt(0);
+            return;
+        }
+        ct.find(a, lane, lo, p.cut_seq, b, s_at);
+    }
+    int T = CT ? a.seq_len : cut ? SsqCut::len(a, b) : min(a.seq_lens[b], a.seq_len);
+    int s_end = s_at + T + p.cut_seq;
+    int t_begin = cut ? SsqCut::token(max(lo, s_at) - s_at, p.cut_seq, T) : split * p.split_len;
+    int t_end = cut ? SsqCut::token(min(hi, s_end) - s_at, p.cut_seq, T) : min(T, t_begin + p.split_len);
+    bool whole = cut ? s_at >= lo && s_end <= hi : p.n_splits == 1;
 
     // ---- prologue: block-table slice, this lane's permutation entries, the query rows (scaled,
     // unpermuted) through LDS into the A registers
@@ -439,7 +485,9 @@ void k_decode_paged_q4(const MfmaParams p) {
 #pragma unroll
     for (int kk = 0; kk < KQ; ++kk) pj[kk] = perm[16 * kk + qj];
     float* qs = reinterpret_cast<float*>(strips);  // [RP][KD] fp32: RP * KD * 4 <= the strips' RP * 512 bytes
-    {
+    float qa[R4][KQ];
+    float qh[R4];  // (unused without passthrough)
+    auto stage_query = [&]() {
         constexpr int kQE = (RP * KD + kThreads - 1) / kThreads;
         int64_t src[kQE];
         bool ok[kQE];
@@ -462,29 +510,28 @@ void k_decode_paged_q4(const MfmaParams p) {
             const int e = tid + k * kThreads;
             if (e < RP * KD) qs[e] = !ok[k] ? 0.f : a.has_scale ? ssq_round_to(qv[k] * a.scale, a.q_dtype) : qv[k];
         }
-    }
-    __syncthreads();  // qs and pages written
-    float qa[R4][KQ];
+        __syncthreads();  // qs and pages written
 #pragma unroll
-    for (int q = 0; q < R4; ++q)
+        for (int q = 0; q < R4; ++q)
 #pragma unroll
-        for (int kk = 0; kk < KQ; ++kk) {
-            qa[q][kk] = qs[(4 * q + qi4) * KD + (int)min((uint64_t)pj[kk], (uint64_t)(KD - 1))];
-            // passthrough blocks score from their stored values (tile_extra_scores): no codeword term
-            if constexpr (HV > 0)
-                if ((a.heavy_mask[0] >> ((16 * kk + qj) / BD)) & 1ull) qa[q][kk] = 0.f;
+            for (int kk = 0; kk < KQ; ++kk) {
+                qa[q][kk] = qs[(4 * q + qi4) * KD + (int)min((uint64_t)pj[kk], (uint64_t)(KD - 1))];
+                // passthrough blocks score from their stored values (tile_extra_scores): no codeword term
+                if constexpr (HV > 0)
+                    if ((a.heavy_mask[0] >> ((16 * kk + qj) / BD)) & 1ull) qa[q][kk] = 0.f;
+            }
+        // the query rows at the passthrough dims: lane 4 j + r holds q_perm[row 4 q + r][hdim[j]] (j < n_hd)
+        if constexpr (HV > 0) {
+            int hd = 0;  // lanes past the last passthrough dim keep dim 0 (their query value is not used)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) hd = j == qj && j < p.n_hd ? p.hdim[j] : hd;
+            const int pd = (int)min((uint64_t)perm[hd], (uint64_t)(KD - 1));
+#pragma unroll
+            for (int q = 0; q < R4; ++q) qh[q] = qj < p.n_hd ? qs[(4 * q + qi4) * KD + pd] : 0.f;
         }
-    // the query rows at the passthrough dims: lane 4 j + r holds q_perm[row 4 q + r][hdim[j]] (j < n_hd)
-    float qh[R4];  // (unused without passthrough)
-    if constexpr (HV > 0) {
-        int hd = 0;  // lanes past the last passthrough dim keep dim 0 (their query value is not used)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) hd = j == qj && j < p.n_hd ? p.hdim[j] : hd;
-        const int pd = (int)min((uint64_t)perm[hd], (uint64_t)(KD - 1));
-#pragma unroll
-        for (int q = 0; q < R4; ++q) qh[q] = qj < p.n_hd ? qs[(4 * q + qi4) * KD + pd] : 0.f;
-    }
-    __syncthreads();  // every wave has its A registers: the strips are free
+        __syncthreads();  // every wave has its A registers: the strips are free
+    };
+    stage_query();
 
     const uint16_t* vbase = reinterpret_cast<const uint16_t*>(a.v) + (int64_t)kv * a.v_sh + (int64_t)(lane & 15) * a.v_st;
     const uint8_t* cbase = PB > 0 ? reinterpret_cast<const uint8_t*>(reinterpret_cast<const uint32_t*>(a.codes) +
@@ -497,8 +544,8 @@ void k_decode_paged_q4(const MfmaParams p) {
                                 : a.codes + (int64_t)b * a.c_sb + (int64_t)kv * a.c_sh + (int64_t)t_begin * a.c_st;
     const uint8_t* vb0 = reinterpret_cast<const uint8_t*>(a.v) +
                          2 * ((int64_t)b * a.v_sb + (int64_t)kv * a.v_sh + (int64_t)t_begin * a.v_st);
-    const int n_tiles = (t_end - t_begin + kTileTok - 1) / kTileTok;
-    const int last_tile = n_tiles > 0 ? n_tiles - 1 : 0;
+    int n_tiles = (t_end - t_begin + kTileTok - 1) / kTileTok;
+    int last_tile = n_tiles > 0 ? n_tiles - 1 : 0;
     TileRegs<NB, DT, PB> RA, RB;
     TileExtra<RP, MK, HV> XA;
     int tile = wave;
@@ -512,20 +559,47 @@ void k_decode_paged_q4(const MfmaParams p) {
         issue_extra<RP, MK, HV, CT>(p, pages, b, kv, t_begin, t_end, min(tile, last_tile), lane, XA);
     }
     (void)RB;
-    // the codebook goes global -> LDS directly: 1 KiB chunks, lane l's 16 bytes at chunk + 16 l;
-    // the tail chunk's lanes past the end re-read the last float4 into the padding
-    {
-        const float* cent = a.cent + (int64_t)kv * a.cent_sh;
-        const int n4 = KD * nc / 4;
-        const int n_chunks = (n4 + 63) / 64;
-        for (int c = wave; c < n_chunks; c += kWaves) {
-            const int i = min(c * 64 + lane, n4 - 1);
-            __builtin_amdgcn_global_load_lds(cent + 4 * i, (__attribute__((address_space(3))) void*)(cb + 256 * c), 16,
-                                             0, 0);
-        }
-    }
+    if (!cut) stage_codebook();
     __builtin_amdgcn_s_waitcnt(0);  // this wave's codebook chunks (and its first tile) have landed
     __syncthreads();
+
+    for (;;) {  // the segments of a share; one pass otherwise
+    // The segment after this one: its block-table entries load beside this one's tiles, and a wave's
+    // last reload here is its first tile there, so the memory stays busy between them.  (That tile's
+    // four entries go through a slice of the wave's own, which needs no barrier.)
+    constexpr int kPgRegs = 2;  // entries per thread held in registers; longer slices finish after the barrier
+    int s_next = 0, e_next = 0, T_next = 0, end_next = 0;
+    bool more = false;
+    int pg[kPgRegs] = {};
+    const int32_t* btab_next = nullptr;
+    const int* pages_next = pages;
+    int tile_next = 0;
+    bool ahead = false;
+    if constexpr (cut) {
+        if (s_end < hi && b + 1 < a.batch) {
+            s_next = s_end;
+            T_next = SsqCut::len(a, b + 1);
+            e_next = s_next + T_next + p.cut_seq;
+            end_next = SsqCut::token(min(hi, e_next) - s_next, p.cut_seq, T_next);
+            more = end_next > 0 || e_next <= hi;  // else: nothing of it but fixed cost
+        }
+        if (more) {
+            btab_next = a.block_table + (int64_t)(b + 1) * a.bt_sb;
+            const int n = (end_next + kPage - 1) / kPage;
+#pragma unroll
+            for (int i = 0; i < kPgRegs; ++i)
+                if (n > 0) pg[i] = btab_next[min(tid + i * kThreads, n - 1)];
+            ahead = n > 0;
+            if (ahead) {
+                tile_next = min(wave, (end_next - 1) / kTileTok);
+                if (lane < 4) first_pg[4 * wave + lane] = btab_next[min(4 * tile_next + lane, n - 1)];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                pages_next = first_pg + 4 * wave - 4 * tile_next;
+            }
+        }
+    }
 
     // ---- stream tiles, two in flight per wave (A/B register sets)
     float m_run[RP], l_lane[RP];
@@ -573,25 +647,42 @@ void k_decode_paged_q4(const MfmaParams p) {
         // one register set: every load is issued unconditionally (clamped to the last tile), so the
         // queue of outstanding loads is the same on every path
         while (tile < n_tiles) {
-            const int next = min(tile + kWaves, last_tile);
+            const bool over = cut && ahead && tile + kWaves >= n_tiles;  // on to the next segment (uniform)
+            const int next = over ? tile_next : min(tile + kWaves, last_tile);
+            const int* npg = over ? pages_next : pages;
+            const int n_begin = over ? 0 : t_begin, n_end = over ? end_next : t_end;
             float s[RP];
             tile_scores_q4<KD, BD, R4, DT, PB>(cb, nc, RA, qa, s);
             tile_extra_scores<R4, MK, HV>(p, qh, XA, s);
-            issue_codes<NB, DT, PB>(a, pages, t_begin, t_end, next, lane, cbase, RA);
-            issue_extra<RP, MK, HV, CT>(p, pages, b, kv, t_begin, t_end, next, lane, XA);
+            issue_codes<NB, DT, PB>(a, npg, n_begin, n_end, next, lane, cbase, RA);
+            issue_extra<RP, MK, HV, CT>(p, npg, b, kv, n_begin, n_end, next, lane, XA);
             tile_softmax_pv<RP, DT, VT, NB, PB>(p, pstrip, b, kv, t_begin + tile * kTileTok, t_end, lane, s, RA, m_run,
                                                 l_lane, acc);
-            issue_values<NB, DT, PB>(a, pages, t_begin, t_end, next, lane, vbase, RA);
+            issue_values<NB, DT, PB>(a, npg, n_begin, n_end, next, lane, vbase, RA);
             tile += kWaves;
+        }
+        if (cut && ahead && wave >= n_tiles) {  // a wave without a tile here
+            issue_tile<NB, DT, PB>(a, pages_next, 0, end_next, tile_next, lane, cbase, vbase, RA);
+            issue_extra<RP, MK, HV, CT>(p, pages_next, b, kv, 0, end_next, tile_next, lane, XA);
         }
     }
 
-    // ---- merge the waves' (m, l, O) through LDS (the codebook is no longer needed)
+    // ---- merge the waves' (m, l, O) through LDS (in the codebook's place where it is done with)
     float l_w[RP];
 #pragma unroll
     for (int r = 0; r < RP; ++r) l_w[r] = wave_sum(l_lane[r]);
-    __syncthreads();
-    float* mbuf = smem;                // [waves][RP]
+    if constexpr (cut) {
+        if (more) {
+            int* next = pages == pages0 ? pages0 + p.cut_pages : pages0;
+            const int n = (end_next + kPage - 1) / kPage;
+#pragma unroll
+            for (int i = 0; i < kPgRegs; ++i)
+                if (tid + i * kThreads < n) next[tid + i * kThreads] = pg[i];
+        }
+    } else {
+        __syncthreads();
+    }
+    float* mbuf = mspace;              // [waves][RP]
     float* lbuf = mbuf + kWaves * RP;  // [waves][RP]
     float* obuf = lbuf + kWaves * RP;  // [waves][RP][Dv]
     constexpr int Dv = DT * 16;
@@ -612,7 +703,15 @@ void k_decode_paged_q4(const MfmaParams p) {
         }
     }
     __syncthreads();
+    if constexpr (cut) {
+        if (more) {  // the rest of the next segment's page slots
+            pages = pages == pages0 ? pages0 + p.cut_pages : pages0;
+            const int n = (end_next + kPage - 1) / kPage;
+            for (int i = tid + kPgRegs * kThreads; i < n; i += kThreads) pages[i] = btab_next[i];
+        }
+    }
     const int n_rows_all = a.batch * a.num_q_heads * a.q_len;
+    if (!cut || whole || t_begin < t_end)  // uniform (a partial segment may hold no token)
     for (int e = tid; e < nr * Dv; e += kThreads) {
         const int r = e / Dv, dv = e - r * Dv;
         float M = -INFINITY;
@@ -628,19 +727,39 @@ void k_decode_paged_q4(const MfmaParams p) {
         const int g = (row0 + r) / a.q_len, qi = row0 + r - g * a.q_len;
         const int h = kv * p.G + g;
         const int rid = (b * a.num_q_heads + h) * a.q_len + qi;
-        if (p.n_splits == 1) {
+        if (whole) {
             ssq_store_elem(a.out, a.v_dtype, (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)qi * a.o_sl + dv, o / L);
             if (a.lse && dv == 0) a.lse[rid] = M + logf(L);
         } else {
-            p.ws_o[((size_t)split * n_rows_all + rid) * Dv + dv] = o;
+            // a share's partials: slot 0 for the sequence it starts in, slot 1 for one it does not finish
+            const size_t at = cut ? (size_t)(2 * bk + (s_at <= lo ? 0 : 1)) * p.rows + r : (size_t)split * n_rows_all + rid;
+            p.ws_o[at * Dv + dv] = o;
             if (dv == 0) {
-                p.ws_m[(size_t)split * n_rows_all + rid] = M;
-                p.ws_l[(size_t)split * n_rows_all + rid] = L;
+                p.ws_m[at] = M;
+                p.ws_l[at] = L;
             }
         }
     }
+    if (!more) break;
+    ++b;
+    s_at = s_next;
+    s_end = e_next;
+    T = T_next;
+    t_begin = 0;
+    t_end = end_next;
+    whole = s_end <= hi;
+    n_tiles = (t_end + kTileTok - 1) / kTileTok;
+    last_tile = n_tiles > 0 ? n_tiles - 1 : 0;
+    tile = wave;
+    stage_query();  // its barriers also end the reads of the merge space and publish the last page slots
+    }
 }
 
+// the instantiations with a length-balanced form: where its merge space fits beside the codebook (up to
+// 4 query rows per KV head, 8 at head_dim 64), without masks or element-wise passthrough loads
+constexpr bool q4_cut(int KD, int R4, bool CT, bool MK, int HV) {
+    return !CT && !MK && HV < 2 && (R4 == 1 || (R4 == 2 && KD == 64));
+}
 
 // waves per workgroup for this instantiation (see k_decode_paged_q4)
 template <int KD, int BD, int R4, int DT>
@@ -649,10 +768,18 @@ constexpr int q4_waves() { return SSQ_Q4_WAVES; }
 template <int KD, int BD, int R4, int DT, int VT, int PB, bool CT, bool MK, int HV>
 int launch_q4(const MfmaParams& mp, const dim3& grid, size_t, hipStream_t st) {
     constexpr int W = q4_waves<KD, BD, R4, DT>();
-    auto kern = k_decode_paged_q4<KD, BD, R4, DT, VT, PB, W, CT, MK, HV>;
+    auto kern = k_decode_paged_q4<KD, BD, R4, DT, VT, PB, W, CT, MK, HV, false>;
+    size_t smem = q4_smem(mp.a, 4 * R4, mp.split_len, W);
+    if (mp.cut_wg) {
+        if constexpr (q4_cut(KD, R4, CT, MK, HV)) {
+            kern = k_decode_paged_q4<KD, BD, R4, DT, VT, PB, W, CT, MK, HV, true>;
+            smem = q4_cut_smem(mp.a, 4 * R4, mp.cut_pages, W);
+        } else {
+            return ssq_fail(SSQ_ERR_UNSUPPORTED, "4x4-MFMA decode: no length-balanced variant");
+        }
+    }
     int rc = ssq_allow_lds((const void*)kern, (int)kMaxSmem, "hipFuncSetAttribute(decode_paged_q4)");
     if (rc) return rc;
-    const size_t smem = q4_smem(mp.a, 4 * R4, mp.split_len, W);
     if (smem > kMaxSmem) return ssq_fail(SSQ_ERR_UNSUPPORTED, "4x4-MFMA decode: %zu bytes of LDS", smem);
     hipLaunchKernelGGL(kern, grid, dim3(W * SSQ_WAVE), smem, st, mp);
     return ssq_check_hip(hipGetLastError(), "k_decode_paged_q4 launch");
