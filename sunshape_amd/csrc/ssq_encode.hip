@@ -150,7 +150,14 @@ extern "C" int ssq_encode(const ssq_encode_args* a, void* stream) {
                         a->kernel);
         const int cw = ssq_code_width(a->n_centroids);
         SSQ_REQUIRE((uintptr_t)a->codes % cw == 0, "%d-bit codes must be %d-byte aligned", 8 * cw, cw);
-        if (a->kernel == 0 && !a->direct_dist && a->block_dim <= 8) return ssq_encode_tile_run(a, st);
+        // The screen stages every codebook once per workgroup and folds its groups, which up to about 2^24
+        // (key, block, codeword) triples costs more than the exact scan split over lanes: bf16 keys of
+        // head_dim 128 over 8 heads, 64 rows at 4,096 codewords of dim 4 (2^23) 18 us on the scan and 34
+        // on the screen, 256 rows at 1,024 of dim 2 (2^24) 12 and 17; 256 at 4,096 (2^25) 30 and 16,
+        // 1,024 at 1,024 (2^26) 28 and 19.  The codes are the same.
+        const int64_t work = (int64_t)a->batch * a->seq_len * a->num_kv_heads * a->n_blocks * a->n_centroids;
+        if (a->kernel == 0 && !a->direct_dist && a->block_dim <= 8 && work > (int64_t)1 << 24)
+            return ssq_encode_tile_run(a, st);
         return ssq_encode_wide_run(a, st);
     }
     if (!a->direct_dist && (a->kernel == 3 || (a->kernel == 0 && a->grid && ssq_encode_grid_supported(a))))

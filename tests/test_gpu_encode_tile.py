@@ -53,9 +53,10 @@ def test_tile_codebooks_past_256(bd, nc):
     values; 16-bit codes."""
     D = 48
     sig, perm, cent = _codec(D, bd, nc, 1, nc)
-    keys = torch.randn(1, 1, 700, D) * sig
+    keys = torch.randn(1, 1, 11000, D) * sig  # more than 2^24 (key, block, codeword) triples: the screen
     for k in (keys.bfloat16(), keys, keys.bfloat16().float(), keys.half()):
         _both(k.to(DEV), perm, cent[0])
+        _both(k[:, :, :700].to(DEV), perm, cent[0])  # the screen or, up to 2^24, the scan
     _both(keys[:, :, :5].to(DEV), perm, cent[0])
 
 
