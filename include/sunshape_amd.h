@@ -129,7 +129,9 @@ typedef struct ssq_decode_args {
     int32_t code_bits;
 } ssq_decode_args;
 
-/* Bytes of device workspace ssq_decode / ssq_attention_scores need (0 if none). */
+/* Bytes of device workspace ssq_decode / ssq_attention_scores need (0 if none).  A paged batch of at
+ * least as many (sequence, KV head) pairs as the device has CUs may ask for one to balance its
+ * workgroups by length; such a call also runs without it, one workgroup per pair. */
 size_t ssq_decode_workspace_size(const ssq_decode_args* a);
 
 /* Fused decode: out = softmax(q.k_hat + mask) @ V per row, plus lse / raw scores on request.
@@ -141,10 +143,11 @@ int ssq_decode(const ssq_decode_args* a, void* workspace, size_t workspace_bytes
  * cannot allocate device memory (code under HIP graph capture, serving loops that forbid
  * hipMalloc).  The caller passes inputs and outputs only; the split workspace ssq_decode would
  * take from the caller lives in a library-owned scratch array of SSQ_NOALLOC_SCRATCH_BYTES per
- * device (held until the process ends).  A problem whose ssq_decode_workspace_size exceeds it
- * fails with SSQ_ERR_UNSUPPORTED before anything is launched.  Calls and results are otherwise
- * those of ssq_decode (same kernels).  Every call on one device shares that device's array:
- * calls that overlap on one device race and must be serialised by the caller. */
+ * device (held until the process ends).  A problem that needs more fails with SSQ_ERR_UNSUPPORTED
+ * before anything is launched.  Batches that ssq_decode balances by length run one workgroup per
+ * (sequence, KV head) pair here, as with num_splits 1, and do not use the array.  Calls and results are
+ * otherwise those of ssq_decode (same kernels).  Every other call on one device shares that device's
+ * array: calls that overlap on one device race and must be serialised by the caller. */
 #define SSQ_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
 int ssq_decode_noalloc(const ssq_decode_args* a, void* stream);
 

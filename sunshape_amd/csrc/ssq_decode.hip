@@ -284,6 +284,7 @@ int ssq_launch_merge(const ssq_decode_args& a, int n_splits, const float* ws_o, 
 
 int ssq_decode_mfma_supported(const ssq_decode_args* a);
 size_t ssq_decode_mfma_workspace(const ssq_decode_args* a);
+size_t ssq_decode_mfma_workspace_least(const ssq_decode_args* a);
 int ssq_decode_mfma(const ssq_decode_args* a, void* workspace, size_t ws_bytes, hipStream_t st);
 int ssq_decode_contig_supported(const ssq_decode_args* a);
 size_t ssq_decode_contig_workspace(const ssq_decode_args* a);
@@ -303,15 +304,21 @@ int pick_kernel(const ssq_decode_args* a) {
 }
 }  // namespace
 
-extern "C" size_t ssq_decode_workspace_size(const ssq_decode_args* a) {
+static size_t workspace_size(const ssq_decode_args* a, bool least) {
     if (validate(a, a && a->v != nullptr) != SSQ_OK) return 0;
     const int k = pick_kernel(a);
-    if (k == 2 && a->v && ssq_decode_mfma_supported(a)) return ssq_decode_mfma_workspace(a);
+    if (k == 2 && a->v && ssq_decode_mfma_supported(a))
+        return least ? ssq_decode_mfma_workspace_least(a) : ssq_decode_mfma_workspace(a);
     if (k == 3 && ssq_decode_contig_supported(a)) return ssq_decode_contig_workspace(a);
     Plan pl;
     if (make_plan(*a, pl) != SSQ_OK) return 0;
     return pl.ws_bytes;
 }
+
+extern "C" size_t ssq_decode_workspace_size(const ssq_decode_args* a) { return workspace_size(a, false); }
+
+// the smallest workspace ssq_decode accepts: that of one workgroup per (sequence, KV head, split)
+size_t ssq_decode_workspace_least(const ssq_decode_args* a) { return workspace_size(a, true); }
 
 extern "C" int ssq_decode(const ssq_decode_args* a, void* workspace, size_t workspace_bytes, void* stream) {
     int rc = validate(a, true);

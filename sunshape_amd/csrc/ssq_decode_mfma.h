@@ -36,6 +36,7 @@ struct SsqMfmaPlan {
     bool q4;           // k_decode_paged_q4 (4x4-MFMA scores) in place of the LUT kernel
     bool ct;           // contiguous rows (the LUT kernel with CT = true)
     size_t smem, ws_bytes;
+    size_t ws_least;   // without length balance, which a call with less workspace than ws_bytes does not get
     int cut_wg, cut_min, cut_seq, cut_pages;  // length-balanced pages (SsqPagedParams)
 };
 

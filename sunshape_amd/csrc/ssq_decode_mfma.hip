@@ -55,6 +55,8 @@ void pt_dims(const ssq_decode_args& a, SsqPagedParams& mp) {
 // segment's prologue and merge (about 4 us at 27 KB/us).  Per call, one workgroup per pair against
 // this, 32/8 heads, head_dim 128, 64 blocks of dim 2: 48 sequences of log-spread lengths up to 8,192, 81 ->
 // 41 us; 64 up to 16,384, 168 -> 79 us; 48 of 8,192 each, 204 -> 177 us; 64 of 4,096 each, 126 -> 123 us.
+// The shares' partials need a workspace where one workgroup per pair needs none, so a call that brings
+// none (ssq_decode_noalloc, whose scratch is shared by every call on a device) runs unbalanced.
 constexpr int kCutSeqBytes = 110 * 1000;
 void plan_cut(const ssq_decode_args& a, int rows, bool pt_vec, SsqMfmaPlan& pl) {
     pl.cut_wg = 0;
@@ -194,6 +196,7 @@ bool plan(const ssq_decode_args* a, SsqMfmaPlan& pl) {
     if (pl.smem > kMaxSmem) return false;
     const size_t n_rows_all = (size_t)a->batch * a->num_q_heads * a->q_len;
     pl.ws_bytes = !nv && pl.n_splits > 1 ? (size_t)pl.n_splits * n_rows_all * (a->value_dim + 2) * 4 : 0;
+    pl.ws_least = pl.ws_bytes;
     plan_cut(*a, rows, dims.pt_vec != 0, pl);
     return true;
 }
@@ -210,10 +213,19 @@ size_t ssq_decode_mfma_workspace(const ssq_decode_args* a) {
     return plan(a, pl) ? pl.ws_bytes : 0;
 }
 
+size_t ssq_decode_mfma_workspace_least(const ssq_decode_args* a) {
+    SsqMfmaPlan pl;
+    return plan(a, pl) ? pl.ws_least : 0;
+}
+
 int ssq_decode_mfma(const ssq_decode_args* a, void* workspace, size_t ws_bytes, hipStream_t st) {
     SsqMfmaPlan pl;
     if (!plan(a, pl)) return ssq_fail(SSQ_ERR_UNSUPPORTED, "MFMA decode kernel does not support this problem");
     if (a->seq_len == 0) return ssq_fail(SSQ_ERR_INVALID, "seq_len == 0: softmax over an empty context");
+    if (pl.cut_wg && (ws_bytes < pl.ws_bytes || !workspace)) {  // no room for the shares' partials
+        pl.cut_wg = 0;
+        pl.ws_bytes = pl.ws_least;
+    }
     SSQ_REQUIRE(ws_bytes >= pl.ws_bytes, "workspace too small: %zu < %zu bytes", ws_bytes, pl.ws_bytes);
     SSQ_REQUIRE(pl.ws_bytes == 0 || workspace, "workspace is NULL");
     MfmaParams mp{};

@@ -6,10 +6,14 @@
 // Every call on one device shares that device's array: calls that overlap on one device (two
 // streams, two threads) race on it and must be serialised by the caller.  The array holds only
 // split partials, which each call writes before it reads them, so nothing in it has to start at
-// zero and no call clears it.
+// zero and no call clears it.  A problem that one workgroup per (sequence, KV head) serves does not
+// touch it: balancing such a batch by length (ssq_decode with a workspace) would share it, so here
+// it runs unbalanced, and calls of that kind may overlap.
 #include "ssq_common.h"
 
 #include <mutex>
+
+size_t ssq_decode_workspace_least(const ssq_decode_args* a);  // ssq_decode.hip
 
 namespace {
 constexpr size_t kScratchBytes = SSQ_NOALLOC_SCRATCH_BYTES;  // per device, held until the process ends
@@ -48,7 +52,7 @@ extern "C" int ssq_decode_noalloc(const ssq_decode_args* a, void* stream) {
     int rc = scratch_on_current_device(&ws);
     if (rc) return rc;
     // 0 for a problem that runs one split per unit, and for invalid arguments (ssq_decode reports them)
-    const size_t need = ssq_decode_workspace_size(a);
+    const size_t need = ssq_decode_workspace_least(a);
     if (need > kScratchBytes)
         return ssq_fail(SSQ_ERR_UNSUPPORTED,
                         "ssq_decode_noalloc: this problem needs %zu bytes of split workspace, more than the "
