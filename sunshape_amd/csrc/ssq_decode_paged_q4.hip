@@ -63,7 +63,8 @@ __global__ __launch_bounds__(256) void k_merge_cut(const SsqPagedParams p) {
         M = Mc;
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] *= f;
-        const uint64_t live = __builtin_amdgcn_ballot_w64(in && wt > 0.f);
+        // every share's values, also at weight 0: 0 times an infinite or NaN value is NaN, as in one pass
+        const uint64_t live = __builtin_amdgcn_ballot_w64(in);
         for (uint64_t t = live; t; t &= t - 1) {
             const int i = __builtin_ctzll(t);
             const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt), i));

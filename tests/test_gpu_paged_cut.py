@@ -101,3 +101,14 @@ def test_cut_graph_replay():
         torch.cuda.synchronize()
         ref, ref_lse = hip_ops.decode(*args, **kw)
         assert torch.equal(out, ref) and torch.equal(lse, ref_lse)
+
+
+def test_cut_infinite_values():
+    """An infinite value under a probability that underflows makes its output NaN (0 times infinity), whichever
+    workgroups the sequence is cut between."""
+    args, kw = _problem([9000] + [3] * 39, 32, 8, 128, 2, 256)
+    args[2][kw["block_table"][0, ::97].long(), :, 5, 3] = float("inf")
+    kw["scale"] = 30.0  # the shares' maxima lie hundreds apart
+    got, ref = hip_ops.decode(*args, **kw), hip_ops.decode(*args, **kw, num_splits=1)
+    assert not torch.isfinite(ref[0][0, :, :, 5]).any()
+    assert torch.equal(torch.isfinite(got[0]), torch.isfinite(ref[0]))
