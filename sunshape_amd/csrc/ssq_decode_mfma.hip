@@ -53,18 +53,28 @@ void pt_dims(const ssq_decode_args& a, SsqPagedParams& mp) {
 // per CU with at least a tile per wave.  The codebook is staged once per workgroup, and a segment's
 // last reloads are the next segment's first tiles.  kCutSeqBytes: what a CU streams during a
 // segment's prologue and merge (about 4 us at 27 KB/us).  Per call, one workgroup per pair against
-// this, 32/8 heads, head_dim 128, 64 blocks of dim 2: 48 sequences of log-spread lengths up to 8,192, 81 ->
-// 41 us; 64 up to 16,384, 168 -> 79 us; 48 of 8,192 each, 204 -> 177 us; 64 of 4,096 each, 126 -> 123 us.
+// this, 32/8 heads, head_dim 128, 64 blocks of dim 2: 48 sequences of log-spread lengths up to 8,192, 79 ->
+// 38 us; 64 up to 8,192, 81 -> 44 us; 48 of 8,192 each, 204 -> 177 us; 64 of 4,096 each, 126 -> 121 us.
+//   Block tables of less than kCutTokens: a cut and the merge's launch cost a batch more than they even
+// out (48 log-spread lengths up to 1,024: 20 -> 26 us).  In longer tables SsqCut decides by the lengths
+// themselves: 64 of 16 tokens 18.4 -> 18.5 us, of 512 33 -> 30; the worst measured, 33 log-spread lengths
+// up to 1,024, 18 -> 21.
+//   KV head counts whose workgroups leave more than 1/16 of the CUs idle (8 sequences of 4,096 tokens
+// with 96 KV heads, 192 workgroups: 189 -> 206 us; 3 with 129: 116 -> 142).
+//   The two slices of block-table entries, for the longest possible segment, leave room for tables of up
+// to about 23,600 tokens at head_dim 128, 256 codewords and 128-dim values; longer tables run unbalanced.
 // The shares' partials need a workspace where one workgroup per pair needs none, so a call that brings
 // none (ssq_decode_noalloc, whose scratch is shared by every call on a device) runs unbalanced.
 constexpr int kCutSeqBytes = 110 * 1000;
+constexpr int kCutTokens = 4096;
 void plan_cut(const ssq_decode_args& a, int rows, bool pt_vec, SsqMfmaPlan& pl) {
     pl.cut_wg = 0;
     if (!pl.q4 || pl.ct || pl.n_groups != 1 || a.num_splits != 0) return;
-    if ((int64_t)a.batch * a.num_kv_heads < ssq_device_cus()) return;
+    const int cus = ssq_device_cus();
+    if ((int64_t)a.batch * a.num_kv_heads < cus || a.seq_len < kCutTokens) return;
     if (!ssq_decode_q4_has_cut(&a, rows) || (a.heavy_mask[0] && !pt_vec)) return;
-    const int n_wg = ssq_device_cus() / a.num_kv_heads;
-    if (n_wg < 1) return;
+    const int n_wg = cus / a.num_kv_heads;
+    if (16 * n_wg * a.num_kv_heads < 15 * cus) return;
     const int token_bytes = a.code_bits == 4 || a.code_bits == 6 ? a.n_blocks / 2 : a.n_blocks;
     const int seq = (kCutSeqBytes / (token_bytes + 2 * a.value_dim) + 63) & ~63;
     const int64_t cost = (int64_t)a.batch * (a.seq_len + seq);

@@ -32,8 +32,14 @@ struct SsqPagedParams {
 // leaves partials, slot 0 of a workgroup for the sequence its share starts in and slot 1 for a later
 // one that it does not finish, which k_merge_cut combines.  Every number here is a function of
 // seq_lens alone, so the decode workgroups and the merge agree without exchanging anything.
+// Where lengths are short or alike, workgroup w takes the sequences w, w + cut_wg, ... whole instead: a
+// cut costs the workgroups on its sides a segment each, which is worth it only if that assignment's
+// fullest workgroup is more than kCutWorth fixed costs over the equal share (64 short sequences in
+// tables of 4,096 tokens: see plan_cut).
+constexpr int kCutWorth = 4;
 struct SsqCut {
     int share, total;
+    bool whole;  // sequences are not cut
     int c0, v0;  // this lane's cost and inclusive sum over the first 64 sequences
     __device__ __forceinline__ static int len(const ssq_decode_args& a, int b) {
         return max(0, min(a.seq_lens[b], a.seq_len));
@@ -64,6 +70,13 @@ struct SsqCut {
         for (int b = SSQ_WAVE; b < a.batch; b += SSQ_WAVE)
             total += __builtin_amdgcn_readlane(scan(cost(a, b + lane, fixed)), 63);
         share = (max((total + n_wg - 1) / n_wg, least) + 63) & ~63;
+        int most = 0;  // the fullest workgroup's cost with whole sequences
+        for (int w = lane; w < n_wg; w += SSQ_WAVE) {
+            int c = 0;
+            for (int b = w; b < a.batch; b += n_wg) c += len(a, b) + fixed;
+            most = max(most, c);
+        }
+        whole = __builtin_amdgcn_ballot_w64(most > share + kCutWorth * fixed) == 0;
     }
     // the sequence that holds cost position x < total, and its start
     __device__ __forceinline__ void find(const ssq_decode_args& a, int lane, int x, int fixed, int& b, int& s) const {

@@ -455,18 +455,20 @@ void k_decode_paged_q4(const MfmaParams p) {
 
     // Length-balanced pages: this workgroup's share [lo, hi) of the cost axis, the sequence at hand and
     // its start on the axis.
-    SsqCut ct{0, 0, 0, 0};
-    int lo = 0, hi = 0, s_at = 0;
+    SsqCut ct{};
+    int lo = 0, hi = 0, s_at = 0, step = 1;
     if (cut) {
         stage_codebook();
         ct.init(a, lane, p.cut_wg, p.cut_seq, p.cut_min);
-        lo = (bk / a.num_kv_heads) * ct.share;
-        hi = lo + ct.share;
-        if (lo >= ct.total) {  // uniform over the workgroup
+        b = bk / a.num_kv_heads;
+        lo = ct.whole ? 0 : b * ct.share;
+        hi = ct.whole ? 0x7fffffff : lo + ct.share;
+        if (ct.whole ? b >= a.batch : lo >= ct.total) {  // uniform over the workgroup
             __builtin_amdgcn_s_waitcnt(0);
             return;
         }
-        ct.find(a, lane, lo, p.cut_seq, b, s_at);
+        if (ct.whole) step = p.cut_wg;  // s_at: the cost of the sequences before, from 0
+        else ct.find(a, lane, lo, p.cut_seq, b, s_at);
     }
     int T = CT ? a.seq_len : cut ? SsqCut::len(a, b) : min(a.seq_lens[b], a.seq_len);
     int s_end = s_at + T + p.cut_seq;
@@ -576,15 +578,15 @@ void k_decode_paged_q4(const MfmaParams p) {
     int tile_next = 0;
     bool ahead = false;
     if constexpr (cut) {
-        if (s_end < hi && b + 1 < a.batch) {
+        if (s_end < hi && b + step < a.batch) {
             s_next = s_end;
-            T_next = SsqCut::len(a, b + 1);
+            T_next = SsqCut::len(a, b + step);
             e_next = s_next + T_next + p.cut_seq;
             end_next = SsqCut::token(min(hi, e_next) - s_next, p.cut_seq, T_next);
             more = end_next > 0 || e_next <= hi;  // else: nothing of it but fixed cost
         }
         if (more) {
-            btab_next = a.block_table + (int64_t)(b + 1) * a.bt_sb;
+            btab_next = a.block_table + (int64_t)(b + step) * a.bt_sb;
             const int n = (end_next + kPage - 1) / kPage;
 #pragma unroll
             for (int i = 0; i < kPgRegs; ++i)
@@ -741,7 +743,7 @@ void k_decode_paged_q4(const MfmaParams p) {
         }
     }
     if (!more) break;
-    ++b;
+    b += step;
     s_at = s_next;
     s_end = e_next;
     T = T_next;
@@ -755,10 +757,12 @@ void k_decode_paged_q4(const MfmaParams p) {
     }
 }
 
-// the instantiations with a length-balanced form: where its merge space fits beside the codebook (up to
-// 4 query rows per KV head, 8 at head_dim 64), without masks or element-wise passthrough loads
+// the instantiations with a length-balanced form: up to 4 query rows per KV head (its merge space fits
+// beside the codebook) at head_dim 128 (at 64 a CU holds two workgroups of the unbalanced form, which
+// measured as fast or faster up to 4,096 tokens: 160 x 2 pairs of 1,024, 27 against 30 us), without masks
+// or element-wise passthrough loads
 constexpr bool q4_cut(int KD, int R4, bool CT, bool MK, int HV) {
-    return !CT && !MK && HV < 2 && (R4 == 1 || (R4 == 2 && KD == 64));
+    return !CT && !MK && HV < 2 && R4 == 1 && KD == 128;
 }
 
 // waves per workgroup for this instantiation (see k_decode_paged_q4)

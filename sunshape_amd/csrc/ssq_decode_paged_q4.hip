@@ -43,6 +43,7 @@ __global__ __launch_bounds__(256) void k_merge_cut(const SsqPagedParams p) {
     const int Dv = a.value_dim;
     SsqCut ct;
     ct.init(a, lane, p.cut_wg, p.cut_seq, p.cut_min);
+    if (ct.whole) return;
     int s, T;
     ct.locate(a, lane, b, p.cut_seq, s, T);
     const int e = s + T + p.cut_seq;

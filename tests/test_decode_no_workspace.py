@@ -39,6 +39,27 @@ print("runs without a workspace")
 """
 
 
+# calls that one workgroup per pair serves as fast or faster: no workspace asked for
+UNBALANCED = """
+a.seq_len = 4095
+assert lib.ssq_decode_workspace_size(ctypes.byref(a)) == 0
+a.seq_len = 8192
+a.batch, a.num_q_heads, a.num_kv_heads = 3, 129 * 4, 129  # one workgroup per KV head: half of the CUs
+assert lib.ssq_decode_workspace_size(ctypes.byref(a)) == 0
+a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim, a.n_blocks, a.value_dim = 160, 14, 2, 64, 32, 64
+assert lib.ssq_decode_workspace_size(ctypes.byref(a)) == 0
+print("unbalanced")
+"""
+
+
+def test_calls_that_are_not_balanced():
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1", CUDA_VISIBLE_DEVICES="-1")
+    abi = os.path.join(HERE, "..", "sunshape_amd", "_abi.py")
+    child = CHILD.split("rc = lib.ssq_decode(")[0] + UNBALANCED
+    r = subprocess.run([sys.executable, "-c", child, N.LIB_PATH, abi], env=env, capture_output=True, text=True, timeout=300)
+    assert "unbalanced" in r.stdout, (r.stdout[-500:], r.stderr[-2000:])
+
+
 def test_balanced_batch_is_not_refused_without_a_workspace():
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1", CUDA_VISIBLE_DEVICES="-1")
     abi = os.path.join(HERE, "..", "sunshape_amd", "_abi.py")
@@ -51,7 +72,7 @@ def test_noalloc_batch_runs_one_workgroup_per_pair():
     """Bit for bit the call with num_splits 1, which has one workgroup per (sequence, KV head) and no
     workspace.  Balanced, sequences cut between workgroups round their probabilities differently."""
     dev, g = "cuda", torch.Generator().manual_seed(1)
-    lens = [3000] + torch.randint(1, 900, (47,), generator=g).tolist()
+    lens = [5000] + torch.randint(1, 900, (47,), generator=g).tolist()
     perm = torch.randperm(128, generator=g).to(dev)
     cent = torch.randn(8, 64, 256, 2, generator=g).to(dev)
     pages = [(n + 15) // 16 for n in lens]
