@@ -18,8 +18,10 @@
 //           from zero (the LUT entry's FMA chain) and is added to the token's scores in block order,
 //           so the raw scores equal the per-token path's bit for bit.
 //   P.V:    A = 16 tokens' probabilities (fp32, from LDS), B = the lane's value element: 2 dims of a
-//           token per lane on contiguous rows, 1 dim of 8 tokens on pages.  A lane keeps Dv / 64 x 4
-//           accumulators, which leaves 16 waves' 128 registers room for the code rows.
+//           token per lane on contiguous rows, 1 dim of 8 tokens on pages.  A lane keeps 2 x 4
+//           accumulators, which leaves 16 waves' 128 registers room for the code rows.  At 64 value dims
+//           a batch takes two 16-token runs, so that as many bytes are in flight as at 128 (16 x 8 x 8,192
+//           tokens, 16 blocks of dim 4, 512 codewords, 4 query rows: pages 81 -> 58 us, rows 60 -> 53).
 //
 // Then per super-tile: mask, optional raw-score store, the softmax update (the super-tile's row
 // maximum), P.V over the super-tile's V rows, and at the end of the split the normalised output +
@@ -29,7 +31,8 @@
 //
 // 1024 threads (16 waves), one workgroup per CU (the double buffer is 128 KiB at 4,096 codewords of
 // dim 4).  4 tokens per thread where a split holds more than 2,048 tokens (a codebook copy per 4,096
-// tokens), 2 below.  32 blocks' codes of each token stay in registers, so a 64-byte row is read once.
+// tokens), 2 below.  32 blocks' codes of each token stay in registers (16 where there are no more), so a
+// 64-byte row is read once.
 //
 // What bounds it, at 32 sequences x 8 KV heads x 16,384 tokens, 4 query rows, 4,096 codewords of dim 4,
 // 128 value dims (1.36 GB; 270 us at a copy's rate): 411 us, of which P.V 146 us (at 7.3 TB/s), the 32
@@ -37,10 +40,11 @@
 // reads out of it and a barrier; 0.84 us at 512 codewords, where the copy is 8 KiB), the rest code rows.
 // 512 threads of 8 tokens with FMA chains on the VALU and rows read 16 bytes at a time took 502 us;
 // 1024 threads of 8 tokens, rows 16 bytes at a time, 437; 512 threads of 8 tokens with whole rows and a
-// block's reads issued under the products of the block before, 505 (too few waves); super-tiles
-// staggered over the sequences, so that one's P.V meets another's blocks, 426 against 395 (a fifth
-// pass costs more than the overlap gives).  Splits of 2,048 tokens: 92 -> 65 us, of 4,096: 136 -> 104.
-// P.V takes 16 tokens per wave and batch: 32 are no faster, 64 on pages 10 to 25 % slower.
+// block's reads issued under the products of the block before, 505 (too few waves).  Super-tiles
+// staggered over the sequences, so that one's P.V meets another's blocks, made an earlier form of this
+// kernel slower, 395 -> 426 (a fifth pass costs more than the overlap gives).  Splits of 2,048 tokens:
+// 92 -> 65 us, of 4,096: 136 -> 104.  At 128 value dims P.V takes 16 tokens per wave and batch: 32 are no
+// faster, 64 on pages 10 to 25 % slower.
 //
 // Host-checked: 16-bit codes in 16-byte aligned rows of a multiple of 8
 // blocks (at most 64), codewords of 2 or 4 dims in a 16-byte aligned codebook of at most 64 KiB per
@@ -115,14 +119,15 @@ __device__ __forceinline__ void stage_block_lds(const float* src_blk, float* hal
 }
 
 // BD: the block dim, 2 or 4 (the plan's condition), fixed at compile time so that each token's
-// codeword is one LDS read and its FMA chain carries no branches.  TPT: tokens per thread.
-template <int RP, bool PAGED, int VT, int BD, int TPT>
+// codeword is one LDS read and its FMA chain carries no branches.  TPT: tokens per thread.  NP: 16-byte
+// pieces of 8 blocks' codes held in registers, 4, or 2 up to 16 blocks.
+template <int RP, bool PAGED, int VT, int BD, int TPT, int NP>
 __global__ __launch_bounds__(kWT) void k_decode_wide(const SsqGenericParams p) {
     extern __shared__ __align__(16) float smem[];
     const ssq_decode_args& a = p.a;
     constexpr int kK = TPT;
     constexpr int kSup = kK * kWT;
-    constexpr int kPieces = 4;  // of 8 blocks' codes in registers
+    constexpr int kPieces = NP;
     const WideLds L = wide_lds(a, RP, TPT);
     const int tid = threadIdx.x;
     const int lane = tid & (SSQ_WAVE - 1);
@@ -356,54 +361,51 @@ __global__ __launch_bounds__(kWT) void k_decode_wide(const SsqGenericParams p) {
         const int nt = min(kSup, t_end - T0);
         const int groups = (nt + 15) >> 4;
         auto probs = [&](int g) {  // 16 tokens' A operand (p past the end is 0)
-            return arow < RP ? pbuf[(size_t)min(arow, RP - 1) * kSup + min(g, groups - 1) * 16 + aj] : 0.f;
+            return arow < RP ? pbuf[(size_t)min(arow, RP - 1) * kSup + g * 16 + aj] : 0.f;
         };
         if (!PAGED) {
             // a lane's 4 bytes are 2 dims: a wave's load is one token's row (128 dims) or two tokens'
             // (64 dims: the lanes' halves take tokens j and j + 8)
-            constexpr int kG = 1;  // groups of 16 tokens per batch
             const uint16_t* vb = reinterpret_cast<const uint16_t*>(a.v) + (int64_t)b * a.v_sb + (int64_t)kv * a.v_sh +
                                  (int64_t)T0 * a.v_st;
             if (Dv == 128) {
-                for (int g0 = wave * kG; g0 < groups; g0 += kWWaves * kG) {
-                    uint32_t raw[kG * 16];
-                    float pa[kG];
+                for (int g = wave; g < groups; g += kWWaves) {
+                    uint32_t raw[16];
 #pragma unroll
-                    for (int k = 0; k < kG * 16; ++k)
+                    for (int k = 0; k < 16; ++k)
                         raw[k] = __builtin_nontemporal_load(
-                            reinterpret_cast<const uint32_t*>(vb + (int64_t)min(g0 * 16 + k, nt - 1) * a.v_st) + lane);
-#pragma unroll
-                    for (int q = 0; q < kG; ++q) pa[q] = g0 + q < groups ? probs(g0 + q) : 0.f;
+                            reinterpret_cast<const uint32_t*>(vb + (int64_t)min(g * 16 + k, nt - 1) * a.v_st) + lane);
+                    const float pa = probs(g);
                     __asm__ volatile("" ::: "memory");  // the batch's loads stay ahead of every use
-                    if ((g0 + kG) * 16 > nt) {  // clamped slots: 0, not p = 0 times a value that may be infinite
+                    if ((g + 1) * 16 > nt) {  // clamped slots: 0, not p = 0 times a value that may be infinite
 #pragma unroll
-                        for (int k = 0; k < kG * 16; ++k) raw[k] = g0 * 16 + k < nt ? raw[k] : 0u;
+                        for (int k = 0; k < 16; ++k) raw[k] = g * 16 + k < nt ? raw[k] : 0u;
                     }
-                    for_each_const<0, kG * 16>([&](auto kc) {
+                    for_each_const<0, 16>([&](auto kc) {
                         constexpr int k = decltype(kc)::value;
-                        acc[0] = mfma4<4, (k & 15)>(pa[k >> 4], val_lo<VT>(raw[k]), acc[0]);
-                        acc[1] = mfma4<4, (k & 15)>(pa[k >> 4], val_hi<VT>(raw[k]), acc[1]);
+                        acc[0] = mfma4<4, k>(pa, val_lo<VT>(raw[k]), acc[0]);
+                        acc[1] = mfma4<4, k>(pa, val_hi<VT>(raw[k]), acc[1]);
                     });
                 }
             } else {
                 const int hl = lane >> 5;
-                for (int g0 = wave * kG; g0 < groups; g0 += kWWaves * kG) {
-                    uint32_t raw[kG * 8];
-                    float pa[kG];
+                for (int g0 = 2 * wave; g0 < groups; g0 += 2 * kWWaves) {  // two groups: as many loads as at 128 dims
+                    uint32_t raw[16];
+                    float pa[2];
 #pragma unroll
-                    for (int k = 0; k < kG * 8; ++k)
+                    for (int k = 0; k < 16; ++k)
                         raw[k] = __builtin_nontemporal_load(
                             reinterpret_cast<const uint32_t*>(
                                 vb + (int64_t)min((g0 + (k >> 3)) * 16 + 8 * hl + (k & 7), nt - 1) * a.v_st) + (lane & 31));
-#pragma unroll
-                    for (int q = 0; q < kG; ++q) pa[q] = g0 + q < groups ? probs(g0 + q) : 0.f;
+                    pa[0] = probs(g0);
+                    pa[1] = g0 + 1 < groups ? probs(g0 + 1) : 0.f;
                     __asm__ volatile("" ::: "memory");
-                    if ((g0 + kG) * 16 > nt) {
+                    if ((g0 + 2) * 16 > nt) {
 #pragma unroll
-                        for (int k = 0; k < kG * 8; ++k)
+                        for (int k = 0; k < 16; ++k)
                             raw[k] = (g0 + (k >> 3)) * 16 + 8 * hl + (k & 7) < nt ? raw[k] : 0u;
                     }
-                    for_each_const<0, kG * 8>([&](auto kc) {
+                    for_each_const<0, 16>([&](auto kc) {
                         constexpr int k = decltype(kc)::value;
                         acc[0] = mfma4<3, (k & 7)>(pa[k >> 3], val_lo<VT>(raw[k]), acc[0]);
                         acc[1] = mfma4<3, (k & 7)>(pa[k >> 3], val_hi<VT>(raw[k]), acc[1]);
@@ -411,59 +413,59 @@ __global__ __launch_bounds__(kWT) void k_decode_wide(const SsqGenericParams p) {
                 }
             }
         } else {
-            // a lane's 16 bytes are 8 tokens of its dim; both halves of a 16-token run and both of the
-            // lane's dims are loaded back to back, so a run's line is fetched once
-            constexpr int kG = 1;
-            const int nd = Dv >> 6;
+            // a lane's 16 bytes are 8 tokens of its dim; both halves of a 16-token run are loaded back to
+            // back, so a run's line is fetched once, and two runs at a time: the run of both of the
+            // lane's dims (128), or two runs of its dim (64; acc[1] then holds the second run's sums)
             const int nchunks = (nt + 7) >> 3;
             const int64_t vhead = (int64_t)kv * a.v_sh + (int64_t)lane * a.v_st;
-            for (int g0 = wave * kG; g0 < groups; g0 += kWWaves * kG) {
-                VRaw8<VT> raw[kG][2][2];  // [group][dim][half]
-                float pa[kG];
+            auto pages_pv = [&](auto two_runs) {
+            constexpr bool two = decltype(two_runs)::value;
+            constexpr int step = two ? 2 : 1;
+            for (int g0 = wave * step; g0 < groups; g0 += kWWaves * step) {
+                VRaw8<VT> raw[2][2];  // [dim or run][half]
+                float pa[2];
+                int64_t src[2][2];
 #pragma unroll
-                for (int q = 0; q < kG; ++q) {
-                    int64_t src[2];
+                for (int e = 0; e < 2; ++e)
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        const int c = min(2 * (g0 + q) + h, nchunks - 1);
+                        const int c = min(2 * (g0 + (two ? e : 0)) + h, nchunks - 1);
                         const int t = T0 + 8 * c;
-                        src[h] = (int64_t)pgl[c] * a.v_sb + vhead + (t - (t / a.page_size) * a.page_size);
+                        src[e][h] = (int64_t)pgl[c] * a.v_sb + vhead + (two ? 0 : 64 * e) * a.v_st +
+                                    (t - (t / a.page_size) * a.page_size);
                     }
 #pragma unroll
-                    for (int e = 0; e < 2; ++e)
+                for (int e = 0; e < 2; ++e)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            raw[q][e][h] = load_v8_raw<VT, true>(a.v, src[h] + (int64_t)(64 * min(e, nd - 1)) * a.v_st);
-                }
-#pragma unroll
-                for (int q = 0; q < kG; ++q) pa[q] = g0 + q < groups ? probs(g0 + q) : 0.f;
+                    for (int h = 0; h < 2; ++h) raw[e][h] = load_v8_raw<VT, true>(a.v, src[e][h]);
+                pa[0] = probs(g0);
+                pa[1] = !two ? pa[0] : g0 + 1 < groups ? probs(g0 + 1) : 0.f;
                 __asm__ volatile("" ::: "memory");
 #pragma unroll
-                for (int q = 0; q < kG; ++q) {
+                for (int e = 0; e < 2; ++e) {
+                    const int g = g0 + (two ? e : 0);
+                    float v[16];
+                    float lo8[8], hi8[8];
+                    unpack_v8<VT>(raw[e][0], lo8);
+                    unpack_v8<VT>(raw[e][1], hi8);
 #pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        if (e < nd) {  // uniform
-                            float v[16];
-                            float lo8[8], hi8[8];
-                            unpack_v8<VT>(raw[q][e][0], lo8);
-                            unpack_v8<VT>(raw[q][e][1], hi8);
-#pragma unroll
-                            for (int j = 0; j < 8; ++j) {
-                                v[j] = lo8[j];
-                                v[8 + j] = hi8[j];
-                            }
-                            if ((g0 + q + 1) * 16 > nt) {  // values of slots past the end are unwritten
-#pragma unroll
-                                for (int j = 0; j < 16; ++j) v[j] = (g0 + q) * 16 + j < nt ? v[j] : 0.f;
-                            }
-                            for_each_const<0, 16>([&](auto jc) {
-                                constexpr int j = decltype(jc)::value;
-                                acc[e] = mfma4<4, j>(pa[q], v[j], acc[e]);
-                            });
-                        }
+                    for (int j = 0; j < 8; ++j) {
+                        v[j] = lo8[j];
+                        v[8 + j] = hi8[j];
                     }
+                    if ((g + 1) * 16 > nt) {  // values of slots past the end are unwritten
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) v[j] = g * 16 + j < nt ? v[j] : 0.f;
+                    }
+                    for_each_const<0, 16>([&](auto jc) {
+                        constexpr int j = decltype(jc)::value;
+                        acc[e] = mfma4<4, j>(pa[e], v[j], acc[e]);
+                    });
                 }
             }
+            };
+            if (Dv == 64) pages_pv(std::true_type{});
+            else pages_pv(std::false_type{});
         }
         __syncthreads();  // p and pgl are read before the next super-tile's stage / pages
     }
@@ -482,6 +484,7 @@ __global__ __launch_bounds__(kWT) void k_decode_wide(const SsqGenericParams p) {
 #pragma unroll
             for (int r = 0; r < RP; ++r) acc[e][r] += __shfl_xor(acc[e][r], 32, SSQ_WAVE);
     }
+    if (PAGED && Dv == 64) acc[0] += acc[1];
     const int d_lane = PAGED ? lane : 2 * (Dv == 64 ? lane & 31 : lane), d_step = PAGED ? 64 : 1;
 #pragma unroll
     for (int e = 0; e < 2; ++e)
@@ -520,7 +523,12 @@ __global__ __launch_bounds__(kWT) void k_decode_wide(const SsqGenericParams p) {
 
 template <int RP, bool PAGED, int VT, int TPT>
 int launch_wide_t(const SsqGenericParams& dp, int n_groups, hipStream_t st) {
-    auto kern = dp.a.block_dim == 4 ? k_decode_wide<RP, PAGED, VT, 4, TPT> : k_decode_wide<RP, PAGED, VT, 2, TPT>;
+    auto kern = k_decode_wide<RP, PAGED, VT, 4, TPT, 4>;
+    if (dp.a.block_dim == 4) {
+        if (dp.a.n_blocks <= 16) kern = k_decode_wide<RP, PAGED, VT, 4, TPT, 2>;
+    } else {
+        kern = dp.a.n_blocks <= 16 ? k_decode_wide<RP, PAGED, VT, 2, TPT, 2> : k_decode_wide<RP, PAGED, VT, 2, TPT, 4>;
+    }
     int rc = ssq_allow_lds((const void*)kern, (int)kMaxSmem, "hipFuncSetAttribute(decode wide)");
     if (rc) return rc;
     const size_t smem = wide_lds(dp.a, RP, TPT).total * sizeof(float);
@@ -548,8 +556,8 @@ int launch_wide_rp(const SsqGenericParams& dp, int n_groups, hipStream_t st) {
                  : launch_wide_tpt<RP, false, SSQ_F16>(dp, n_groups, st);
 }
 
-// rows per workgroup: 1, or 4 for 2 to 4 (the matrix-core blocks hold 4 rows either way)
-int wide_rows(int RP) { return RP == 1 ? 1 : 4; }
+// rows per workgroup: 1, 2 or 4 (the matrix-core blocks hold 4 rows either way; the softmax does not)
+int wide_rows(int RP) { return RP <= 2 ? RP : 4; }
 
 }  // namespace
 
@@ -566,5 +574,9 @@ bool ssq_decode_wide_fits(const ssq_decode_args& a) {
 }
 
 int ssq_decode_wide(const SsqGenericParams& dp, int RP, int n_groups, size_t, hipStream_t st) {
-    return wide_rows(RP) == 1 ? launch_wide_rp<1>(dp, n_groups, st) : launch_wide_rp<4>(dp, n_groups, st);
+    switch (wide_rows(RP)) {
+        case 1: return launch_wide_rp<1>(dp, n_groups, st);
+        case 2: return launch_wide_rp<2>(dp, n_groups, st);
+        default: return launch_wide_rp<4>(dp, n_groups, st);
+    }
 }

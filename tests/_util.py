@@ -1,6 +1,6 @@
 """Helpers shared by the GPU parity tests.
 
-Tolerances (north-star): fp32 scores within 1e-4 and bf16 outputs within 2e-2,
+Tolerances: fp32 scores within 1e-4 and bf16 outputs within 2e-2,
 measured norm-relative: max|got - ref| <= tol * max|ref| over the compared tensor.
 Encode indices are compared bit-for-bit.
 """
@@ -46,3 +46,23 @@ def bf16_from_bits(bits) -> np.ndarray:
 
 def torch_bf16_from_bits(bits, device) -> torch.Tensor:
     return torch.from_numpy(np.asarray(bits).astype(np.int16)).view(torch.bfloat16).to(device)
+
+
+def time_us(fn):
+    """The fastest of five replays of eight captured calls, per call."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(8):
+            fn()
+    graph.replay()
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1000 / 8)
+    return best

@@ -14,6 +14,8 @@ import torch
 
 from sunshape_amd import hip_ops
 
+from _util import time_us
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -24,6 +26,9 @@ DEV = "cuda"
     (80, 2, 512, 64, 3, True, torch.float16),       # 40 blocks: the second part has one piece
     (96, 4, 4096, 128, 1, True, torch.bfloat16),    # 24 blocks, one query row
     (32, 4, 2048, 64, 2, False, torch.float16),     # 8 blocks
+    (64, 4, 512, 64, 4, True, torch.bfloat16),      # 16 blocks, pages of 64 value dims: two 16-token runs
+    (64, 4, 512, 64, 2, False, torch.bfloat16),     # at a time, as contiguous rows of 64 dims
+    (32, 2, 512, 64, 2, True, torch.float16),       # two query rows
 ])
 def test_row_pieces_and_tails(D, bd, nc, Dv, Hq, paged, dtype, T, splits):
     g = torch.Generator().manual_seed(T + D)
@@ -57,3 +62,22 @@ def test_row_pieces_and_tails(D, bd, nc, Dv, Hq, paged, dtype, T, splits):
     assert torch.isfinite(out).all()
     assert float((out.float() - ref.float()).abs().max()) <= 2.0 ** -8 * float(ref.float().abs().max())
     assert float((lse - lse_r).abs().max()) <= 1e-6 * float(lse_r.abs().max())
+
+
+@pytest.mark.parametrize("Hq", [8, 32])
+def test_pages_time_at_64_dims(Hq):
+    """Pages of 64 value dims take at most 1.25 times the contiguous rows' time (1.08 to 1.13; with one 16-token run
+    loaded at a time, 1.35 to 1.42)."""
+    B, Hkv, T, D, bd, nc = 16, 8, 8192, 64, 4, 512
+    gd = torch.Generator(device=DEV).manual_seed(5)
+    perm = torch.randperm(D, generator=gd, device=DEV)
+    cent = torch.randn(Hkv, D // bd, nc, bd, generator=gd, device=DEV)
+    q = torch.randn(B, Hq, 1, D, generator=gd, device=DEV, dtype=torch.bfloat16)
+    codes = torch.randint(0, nc, (B, Hkv, T, D // bd), generator=gd, device=DEV, dtype=torch.int16)
+    v = torch.randn(B, Hkv, T, D, generator=gd, device=DEV, dtype=torch.bfloat16)
+    table = torch.randperm(B * T // 16, generator=gd, device=DEV).view(B, T // 16).to(torch.int32)
+    lens = torch.full((B,), T, dtype=torch.int32, device=DEV)
+    rows = time_us(lambda: hip_ops.decode(q, codes, v, perm, cent, scale=0.125))
+    cp, vp = codes.view(B * T // 16, Hkv, 16, D // bd), v.view(B * T // 16, Hkv, D, 16)
+    pages = time_us(lambda: hip_ops.decode(q, cp, vp, perm, cent, scale=0.125, block_table=table, seq_lens=lens))
+    assert pages < 1.25 * rows, (pages, rows)
