@@ -191,8 +191,9 @@ typedef struct ssq_encode_args {
     void* pt; int32_t pt_dtype; int32_t pt_dense; int64_t pt_sb, pt_sh, pt_st;
     const int64_t* slot_mapping; int64_t sm_sb; int32_t page_size;
     int32_t kernel;      /* 0 auto, 1 VALU exact scan, 2 MFMA screen + exact certification, 3 grid search
-                            (2 and 3 serve at most 256 codewords; more run the MFMA screen under 0 up to
-                            block_dim 8, else the exact scan over LDS chunks of the codebook) */
+                            (2 and 3 serve at most 256 codewords; more run the exact scan over LDS chunks
+                            of the codebook, or under 0, for block_dim 3 to 8 and all but small calls,
+                            the MFMA screen) */
     const void* grid; uint64_t grid_bytes;  /* optional search grid from ssq_encode_grid_build (or NULL) */
     /* 1: torch.cdist's direct evaluation, sqrt(sum_k (x_k - c_k)^2) with the rounded squares summed
      * in k order, which torch takes in place of the mm formulation when both of its inputs have at

@@ -170,7 +170,7 @@ int ssq_device_cus();
 bool ssq_encode_grid_supported(const ssq_encode_args* a);
 int ssq_encode_grid_run(const ssq_encode_args* a, hipStream_t st);
 // matrix-core screen + exact evaluation (ssq_encode_tile.hip): 256 codewords, or more than 256 with
-// block dims up to 8
+// block dims 3 to 8
 int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st);
 // exact scan for codebooks of more than 256 codewords (ssq_encode_wide.hip)
 int ssq_encode_wide_run(const ssq_encode_args* a, hipStream_t st);

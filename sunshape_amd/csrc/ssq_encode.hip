@@ -146,17 +146,22 @@ extern "C" int ssq_encode(const ssq_encode_args* a, void* stream) {
                     "direct_dist runs on the exact scan (kernel 0 or 1), not kernel %d", a->kernel);
     if (a->n_centroids > 256) {  // 16- / 32-bit codes
         SSQ_UNSUPPORTED(a->kernel == 0 || a->kernel == 1,
-                        "n_centroids=%d encodes on the exact scan (kernel 0 or 1), not kernel %d", a->n_centroids,
+                        "n_centroids=%d encodes under kernel 0, or 1 for the exact scan, not kernel %d", a->n_centroids,
                         a->kernel);
         const int cw = ssq_code_width(a->n_centroids);
         SSQ_REQUIRE((uintptr_t)a->codes % cw == 0, "%d-bit codes must be %d-byte aligned", 8 * cw, cw);
-        // The screen stages every codebook once per workgroup and folds its groups, which up to about 2^24
-        // (key, block, codeword) triples costs more than the exact scan split over lanes: bf16 keys of
-        // head_dim 128 over 8 heads, 64 rows at 4,096 codewords of dim 4 (2^23) 18 us on the scan and 34
-        // on the screen, 256 rows at 1,024 of dim 2 (2^24) 12 and 17; 256 at 4,096 (2^25) 30 and 16,
-        // 1,024 at 1,024 (2^26) 28 and 19.  The codes are the same.
-        const int64_t work = (int64_t)a->batch * a->seq_len * a->num_kv_heads * a->n_blocks * a->n_centroids;
-        if (a->kernel == 0 && !a->direct_dist && a->block_dim <= 8 && work > (int64_t)1 << 24)
+        // The screen stages every codebook once per 512 keys of a KV head and folds its groups, which for few
+        // keys, and up to about 2^24 (key, block, codeword) triples, costs more than the exact scan split
+        // over lanes: bf16 keys of head_dim 128 over 8 heads, 64 rows at 4,096 codewords of dim 4 (2^23)
+        // 18 us on the scan and 34 on the screen, 8 at 65,535 (2^27) 215 and 454.  Codebooks of dims 1 and 2
+        // stay on the scan: many codewords then lie within the screen's bound of the nearest, which leaves
+        // most pairs to a scan of its own (2,048 keys at 1,024 codewords of dim 1: 303 us on the scan, 612
+        // on the screen; 4,096 at 1,024 of dim 2, 323 and 136 when centred, 590 with an offset of 30 standard
+        // deviations).  The codes are the same.
+        const int64_t keys = (int64_t)a->batch * a->seq_len;
+        const int64_t work = keys * a->num_kv_heads * a->n_blocks * a->n_centroids;
+        if (a->kernel == 0 && !a->direct_dist && a->block_dim >= 3 && a->block_dim <= 8 && keys >= 32 &&
+            work > (int64_t)1 << 24)
             return ssq_encode_tile_run(a, st);
         return ssq_encode_wide_run(a, st);
     }

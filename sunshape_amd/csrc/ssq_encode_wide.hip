@@ -3,9 +3,8 @@
 // (sunshape/codec.py:78-83; SunShapeBlockCodec.quantize, :362-385).  The reference's default
 // fitter gives such codebooks at bits_per_dim * block_dim > 8 (n_centroids = 2^round(bits * bd),
 // sunshape/hf.py:594): 4,096 codewords at 3 bits/dim and block_dim 4.  This exact scan
-// serves kernel 1, the direct distance and block_dim above 8; the rest take the matrix-core screen
-// (ssq_encode_tile.hip, same codes: a round trip of 65,536 fp32 keys at 4,096 codewords of dim 4 takes
-// 403 us with it, 1,440 with this scan).
+// serves kernel 1, the direct distance, block dims below 3 and above 8, and small calls (the rule is in
+// ssq_encode.hip); the rest take the matrix-core screen (ssq_encode_tile.hip, same codes).
 //
 // One thread per (key, block), one light block per workgroup (blockIdx.z); the block's codewords
 // pass through LDS in chunks (in the metric space E_b c under a SunShape-Pro metric) with their

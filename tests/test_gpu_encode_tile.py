@@ -10,6 +10,8 @@ import torch
 
 from sunshape_amd import hip_ops
 
+from _util import time_us
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -20,6 +22,13 @@ def _codec(D, bd, nc, heads, seed):
     perm = torch.randperm(D, generator=g)
     cent = torch.randn(heads, D // bd, nc, bd, generator=g) * sig[perm].view(D // bd, 1, bd)
     return sig, perm.to(DEV), cent.to(DEV)
+
+
+def _screened(keys, cent):
+    """Whether a call past 256 codewords takes the screen: block dims 3 to 8, at least 32 keys per KV head and
+    more than 2^24 (key, block, codeword) triples."""
+    n = keys.shape[0] * keys.shape[2]
+    return cent.shape[-1] >= 3 and n >= 32 and n * keys.shape[1] * cent.shape[-3] * cent.shape[-2] > 1 << 24
 
 
 def _both(keys, perm, cent, **kw):
@@ -41,11 +50,11 @@ def test_tile_key_counts_and_block_dims(bd, D, dtype):
         keys = (torch.randn(B, 2, S, D, generator=g) * sig).to(dtype).to(DEV)
         _both(keys, perm, cent)
     odd = torch.empty(1, 2, 300, D + 1, dtype=dtype, device=DEV)[..., :D]  # rows off 16-byte alignment
-    odd.copy_((torch.randn(1, 2, 300, D) * sig).to(dtype))
+    odd.copy_((torch.randn(1, 2, 300, D, generator=g) * sig).to(dtype))
     _both(odd, perm, cent)
 
 
-@pytest.mark.parametrize("bd", [2, 3, 4, 8])
+@pytest.mark.parametrize("bd", [3, 4, 8])
 @pytest.mark.parametrize("nc", [257, 512, 1023, 1025, 2500])
 def test_tile_codebooks_past_256(bd, nc):
     """Codebooks that end inside, at and just past a 1,024- or 512-codeword stage, and one codeword
@@ -53,11 +62,14 @@ def test_tile_codebooks_past_256(bd, nc):
     values; 16-bit codes."""
     D = 48
     sig, perm, cent = _codec(D, bd, nc, 1, nc)
-    keys = torch.randn(1, 1, 11000, D) * sig  # more than 2^24 (key, block, codeword) triples: the screen
+    keys = torch.randn(1, 1, 11000, D, generator=torch.Generator().manual_seed(nc + bd)) * sig
+    least = (1 << 24) // (D // bd * nc) + 1  # the smallest call on the screen
     for k in (keys.bfloat16(), keys, keys.bfloat16().float(), keys.half()):
-        _both(k.to(DEV), perm, cent[0])
-        _both(k[:, :, :700].to(DEV), perm, cent[0])  # the screen or, up to 2^24, the scan
-    _both(keys[:, :, :5].to(DEV), perm, cent[0])
+        for n in (11000, least):
+            assert _screened(k[:, :, :n], cent)
+            _both(k[:, :, :n].to(DEV), perm, cent[0])
+    assert not _screened(keys[:, :, :least - 1], cent)  # the last call on the scan, split over lanes
+    _both(keys[:, :, :least - 1].to(DEV), perm, cent[0])
 
 
 @pytest.mark.parametrize("nc", [256, 700])
@@ -77,7 +89,9 @@ def test_tile_ties_and_extreme_codebooks(nc, ties):
         cent[5, 200] = float("inf")
     else:
         cent[2] *= 1e19
-    keys = torch.randn(1, 1, 700, D) * sig
+    n = 700 if nc == 256 else 1600  # past 256 codewords: enough for the screen
+    keys = torch.randn(1, 1, n, D, generator=torch.Generator().manual_seed(n)) * sig
+    assert nc == 256 or _screened(keys, cent)
     keys[0, 0, 5] = 1e25
     keys[0, 0, 6, 3] = float("nan")
     keys[0, 0, 7] = 0
@@ -90,17 +104,33 @@ def test_tile_heavy_pages_metric_and_repeated_dims(nc):
     block metric, and a permutation that repeats a dim (gathered, not inverted)."""
     D, bd, B, S = 128, 4, 5, 130
     sig, perm, cent = _codec(D, bd, nc, 2, 11)
-    keys = (torch.randn(B, 2, S, D) * sig).bfloat16().to(DEV)
+    g = torch.Generator().manual_seed(nc)
+    keys = (torch.randn(B, 2, S, D, generator=g) * sig).bfloat16().to(DEV)
+    assert nc == 256 or _screened(keys, cent)
     heavy = [b in (0, 9, 31) for b in range(D // bd)]
     _both(keys, perm, cent, heavy=heavy)
     _both(keys, perm, cent, heavy=heavy, pt_dense=True, pt_dtype=torch.float32)
-    E = (torch.eye(D) + 0.2 * torch.randn(D, D)).to(DEV)
+    E = (torch.eye(D) + 0.2 * torch.randn(D, D, generator=g)).to(DEV)
     _both(keys, perm, cent, metric=E)
     rep = perm.clone()
     rep[3] = rep[90]
     _both(keys, rep, cent)
-    slots = torch.randperm(B * S, device=DEV).view(B, S)
+    slots = torch.randperm(B * S, generator=g).view(B, S).to(DEV)
     pages = [torch.zeros((B * S + 15) // 16, 2, 16, D // bd, dtype=hip_ops.index_dtype(nc), device=DEV) for _ in range(2)]
     for out, kernel in zip(pages, (0, 1)):
         hip_ops.encode(keys, perm, cent, codes_out=out, slot_mapping=slots, kernel=kernel)
     assert torch.equal(pages[0], pages[1])
+
+
+def _offset_problem(n, H, D, bd, nc, dtype, off):
+    g = torch.Generator(device=DEV).manual_seed(1)
+    perm = torch.randperm(D, generator=g, device=DEV)
+    cent = torch.randn(H, D // bd, nc, bd, generator=g, device=DEV) + off
+    return (torch.randn(1, H, n, D, generator=g, device=DEV) + off).to(dtype), perm, cent
+
+
+@pytest.mark.parametrize("n,H,D,bd,nc", [(1024, 1, 128, 2, 300), (2048, 8, 128, 1, 1024), (8, 8, 128, 4, 65535)])
+def test_wide_calls_that_stay_on_the_scan(n, H, D, bd, nc):
+    """Few keys, and codebooks of dims 1 and 2: the exact scan serves them faster than the screen (2 to 6 times)."""
+    a = _offset_problem(n, H, D, bd, nc, torch.bfloat16, 0.0)
+    assert time_us(lambda: hip_ops.encode(*a)) < 1.3 * time_us(lambda: hip_ops.encode(*a, kernel=1))

@@ -100,8 +100,9 @@ def _merge_codebook(seed, nb, nc, bd, n):
 def test_wide_encode_sqrt_merges(n, direct):
     """4,096 codewords of dim 4 built so that sqrt merges are common (the first argmin of the
     distance has a larger pre-sqrt value than another codeword in hundreds of (key, block) pairs):
-    bit-exact with the oracle with one lane per scan (66,000 keys), split scans (2,000 keys) and
-    torch.cdist's direct distance (20 keys)."""
+    bit-exact with the oracle on the matrix-core screen (kernel 0 at 66,000 and 2,000 keys), on the
+    exact scan with one lane per scan (kernel 1, 66,000 keys) and split scans (kernel 1, 2,000 keys),
+    and with torch.cdist's direct distance (20 keys)."""
     log(f"wide encode sqrt merges n={n} direct={direct}")
     nb, nc, bd = 4, 4096, 4
     cent, x = _merge_codebook(11 + n, nb, nc, bd, n)
@@ -114,10 +115,12 @@ def test_wide_encode_sqrt_merges(n, direct):
     if n >= 2000:
         assert keep > 50, keep  # the construction reaches the tie cases it is for
     ref, _ = O.encode(x, perm, cent, direct=direct, threads=8)
-    codes, _ = hip_ops.encode(torch.from_numpy(x)[None, None].to(DEV), torch.from_numpy(perm)[None].to(DEV),
-                              torch.from_numpy(cent)[None].to(DEV), direct=direct)
-    got = _idx(codes)[0, 0]
-    assert np.array_equal(got, ref.astype(np.int64)), int((got != ref.astype(np.int64)).sum())
+    assert direct or n * nb * nc > 1 << 24  # kernel 0 takes the screen
+    for kernel in (0, 1):
+        codes, _ = hip_ops.encode(torch.from_numpy(x)[None, None].to(DEV), torch.from_numpy(perm)[None].to(DEV),
+                                  torch.from_numpy(cent)[None].to(DEV), direct=direct, kernel=kernel)
+        got = _idx(codes)[0, 0]
+        assert np.array_equal(got, ref.astype(np.int64)), (kernel, int((got != ref.astype(np.int64)).sum()))
 
 
 @pytest.mark.parametrize("nc,bd", [(4096, 4), (65536, 2)])
