@@ -103,14 +103,15 @@ constexpr int slot_dwords(int bdp, bool raw16) { return raw16 ? bdp / 2 : bdp; }
 constexpr int kOpenCap = 512;
 
 // LDS: operands [2][kOps] | (one stage only: records [2][kRecs]) | bad [nbc], two-part flag, open
-//      count | slot of block [128] | heavy blocks [128] | open pairs [kOpenCap] u16 | keys [nbc + 1][kKeyRow][slot dwords] (the last slot takes
+//      count | slot of block [128] | heavy blocks [128] | open pairs [kOpenCap] u16 | (under a
+//      metric: E_b [nbc][BDP][BDP]) | keys [nbc + 1][kKeyRow][slot dwords] (the last slot takes
 //      the dims of other chunks and of heavy blocks where rows load whole; block dims 9 and 10 are
 //      always gathered and have none)
 template <int BDP, bool WIDE>
-size_t tile_smem(int nbc, bool raw16) {
+size_t tile_smem(int nbc, bool raw16, const ssq_encode_args& a) {
     using Sh = TileShape<BDP, WIDE>;
     const size_t dw = 2 * (size_t)Sh::kOps + 2 * (size_t)Sh::kRecs + (size_t)((nbc + 5) & ~3) + 64 + kOpenCap / 2;
-    return (dw + (size_t)(nbc + (BDP < 16 ? 1 : 0)) * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
+    return (dw + (a.metric ? (size_t)nbc * BDP * BDP : 0) + (size_t)(nbc + (BDP < 16 ? 1 : 0)) * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
 }
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
@@ -229,20 +230,15 @@ __device__ __forceinline__ void load_row(const float* cent, uint32_t j, int bd, 
         for (int d = 0; d < BDP; ++d) c[d] = d < bd ? c[d] : 0.f;
     }
 }
-// y_k = sum_j E_b[k][j] v_j (metric_row's order), in place
+// y_k = sum_j E_b[k][j] v_j (metric_row's order), in place; eb: E_b in LDS, zero-padded like v
 template <int BDP>
-__device__ __forceinline__ void to_metric(const float* eb, int D, int bd, float (&v)[BDP]) {
+__device__ __forceinline__ void to_metric(const float* eb, float (&v)[BDP]) {
     float y[BDP];
 #pragma unroll
     for (int k = 0; k < BDP; ++k) {
-        float acc = 0.f;
-        if (k < bd) {
-            acc = eb[(int64_t)k * D] * v[0];
+        y[k] = eb[k * BDP] * v[0];
 #pragma unroll
-            for (int j = 1; j < BDP; ++j)
-                if (j < bd) acc = __builtin_fmaf(eb[(int64_t)k * D + j], v[j], acc);
-        }
-        y[k] = acc;
+        for (int j = 1; j < BDP; ++j) y[k] = __builtin_fmaf(eb[k * BDP + j], v[j], y[k]);
     }
 #pragma unroll
     for (int k = 0; k < BDP; ++k) v[k] = y[k];
@@ -293,7 +289,8 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     uint8_t* blkslot = reinterpret_cast<uint8_t*>(bad + ((p.nbc + 5) & ~3));
     uint8_t* heavyL = blkslot + 128;
     u16a* open_list = reinterpret_cast<u16a*>(heavyL + 128);
-    u32a* keysL = reinterpret_cast<u32a*>(open_list + kOpenCap);
+    float* metL = reinterpret_cast<float*>(open_list + kOpenCap);  // [nl][BDP][BDP]
+    u32a* keysL = reinterpret_cast<u32a*>(open_list + kOpenCap) + (a.metric ? p.nbc * BDP * BDP : 0);
     u32a* mykeys = keysL + (wave * 32) * SD;  // slot j of key m: mykeys + (j * kKeyRow + m) * SD
 
     for (int j = tid; j <= p.nbc + 1; j += kTileThreads) bad[j] = 0;  // and *two_part, *n_open
@@ -308,6 +305,14 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     const float* cent = a.cent + (int64_t)kv * a.cent_sh;
     const int64_t* perm = a.perm + (int64_t)kv * a.perm_sh;
     const float* met = a.metric ? a.metric + (int64_t)kv * a.metric_sh : nullptr;
+
+    if (met) {  // the chunk's diagonal blocks of the metric
+        for (int i = tid; i < nl * BDP * BDP; i += kTileThreads) {
+            const int r = i / BDP % BDP, c = i % BDP;
+            const int64_t o = p.light[l0 + i / (BDP * BDP)] * bd;
+            metL[i] = r < bd && c < bd ? met[(o + r) * D + o + c] : 0.f;
+        }
+    }
 
     // output rows of this lane's key, and the row of its elements
     int64_t crow = 0, prow = 0, krow = 0;
@@ -440,6 +445,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         }
         wave_sync_lds();
     }
+    if (met) __syncthreads();  // metL
     if (KM == kKeyF32 && met && live) {  // the key blocks' images under the block metric
         low = 0;
         for (int j = half; j < nl; j += 2) {
@@ -448,8 +454,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
             float x[BDP];
             lds_dwords<SD>(ks, kw);
             slot_elems<BDP, KM>(kw, x);
-            const int blk = p.light[l0 + j];
-            to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, x);
+            to_metric<BDP>(metL + j * BDP * BDP, x);
 #pragma unroll
             for (int d = 0; d < BDP; ++d) {
                 ks[d] = __float_as_uint(x[d]);
@@ -485,10 +490,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     // operand dword i of a codeword, from its row's first dword: [MFMA][half][row][4 dwords]
     constexpr auto at_dw = [](int i) { return (i / 8) * 256 + ((i / 4) & 1) * 128 + (i & 3); };
     auto store_cw = [&](int it, int j, int st) {
-        if (met) {
-            const int blk = p.light[l0 + j];
-            to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, cw);
-        }
+        if (met) to_metric<BDP>(metL + j * BDP * BDP, cw);
         const float cn = norm_p<BDP>(cw);
         if (!(cn < 0x1.0p120f)) bad[j] = 1;
         uint32_t kd[8 * NM];
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
             for (int i = 0; i < NB; ++i) load_row<BDP>(cb, min(n0 + 64 * i, nc - 1), bd, p.vec, c[i]);
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
-                if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[i]);
+                if (met) to_metric<BDP>(metL + j * BDP * BDP, c[i]);
                 // past the end: the last codeword again, which cannot win over itself
                 take_min(exact_e<BDP>(xm, xmn, c[i], norm_p<BDP>(c[i])), (uint32_t)min(n0 + 64 * i, nc - 1), be, bn);
             }
@@ -725,7 +727,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                     for (int i = 0; i < NC; ++i) load_row<BDP>(cb, min(first + i, nc - 1), bd, p.vec, c[i]);
 #pragma unroll
                     for (int i = 0; i < NC; ++i) {
-                        if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[i]);
+                        if (met) to_metric<BDP>(metL + j * BDP * BDP, c[i]);
                         const float e = exact_e<BDP>(m2x, xn, c[i], norm_p<BDP>(c[i]));
                         best[i] = {first + i < nc ? __float_as_int(e) : kInfBits, kInfBits, i};
                     }
@@ -806,7 +808,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                 for (int u = 0; u < NB; ++u) load_row<BDP>(cb, min(n0 + 16 * u, nc - 1), bd, p.vec, c[u]);
 #pragma unroll
                 for (int u = 0; u < NB; ++u) {
-                    if (met) to_metric<BDP>(met + (int64_t)(blk * bd) * D + blk * bd, D, bd, c[u]);
+                    if (met) to_metric<BDP>(metL + j * BDP * BDP, c[u]);
                     take_min(exact_e<BDP>(xm, xmn, c[u], norm_p<BDP>(c[u])), (uint32_t)min(n0 + 16 * u, nc - 1), be, bn);
                 }
             }
@@ -882,7 +884,7 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     const ssq_encode_args& a = tp.a;
     constexpr bool raw16 = KM != kKeyF32;
     int nbc = tp.n_light > 0 ? tp.n_light : 1;
-    while (nbc > 1 && tile_smem<BDP, WIDE>(nbc, raw16) > kTileSmemCap) --nbc;
+    while (nbc > 1 && tile_smem<BDP, WIDE>(nbc, raw16, a) > kTileSmemCap) --nbc;
     tp.fold = ssq_encode_fold(&a, kTileKeys);
     const int64_t n_keys = tp.fold ? (int64_t)a.batch * a.seq_len : a.seq_len;
     const int64_t xg = (n_keys + kTileKeys - 1) / kTileKeys;
@@ -918,7 +920,7 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     SSQ_UNSUPPORTED(groups <= 0x7fffffff && wgs <= 0x7fffffff, "too many keys for one encode launch");
     tp.xg = (int)xg;
     tp.groups = (int)groups;
-    const size_t smem = tile_smem<BDP, WIDE>(nbc, raw16);
+    const size_t smem = tile_smem<BDP, WIDE>(nbc, raw16, a);
     SSQ_UNSUPPORTED(smem <= kTileSmemCap, "block too large for the MFMA encode");
     const int rc = ssq_allow_lds((const void*)k_encode_tile<BDP, KM, WIDE>, (int)kTileSmemCap,
                                  "hipFuncSetAttribute(encode tile)");
