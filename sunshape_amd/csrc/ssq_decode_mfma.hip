@@ -57,8 +57,8 @@ void pt_dims(const ssq_decode_args& a, SsqPagedParams& mp) {
 // 38 us; 64 up to 8,192, 81 -> 44 us; 48 of 8,192 each, 204 -> 177 us; 64 of 4,096 each, 126 -> 121 us.
 //   Block tables of less than kCutTokens: a cut and the merge's launch cost a batch more than they even
 // out (48 log-spread lengths up to 1,024: 20 -> 26 us).  In longer tables SsqCut decides by the lengths
-// themselves: 64 of 16 tokens 18.4 -> 18.5 us, of 512 33 -> 30; the worst measured, 33 log-spread lengths
-// up to 1,024, 18 -> 21.
+// themselves: 64 of 16 tokens 18.4 -> 18.5 us, of 512 33 -> 30 (16 codewords: 16.7 -> 17.8, the merge's
+// launch); the worst measured, 33 log-spread lengths up to 1,024, 18 -> 24.
 //   KV head counts whose workgroups leave more than 1/16 of the CUs idle (8 sequences of 4,096 tokens
 // with 96 KV heads, 192 workgroups: 189 -> 206 us; 3 with 129: 116 -> 142).
 //   The two slices of block-table entries, for the longest possible segment, leave room for tables of up

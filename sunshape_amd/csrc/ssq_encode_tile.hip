@@ -3,15 +3,19 @@
 // reference's winner, and the reference's own fp32 arithmetic decides inside it.  Serves 256-codeword
 // codebooks (kernel 2) and, with the codebook streamed through LDS, codebooks past 256 codewords.
 //
-// Screen.  v_mfma_f32_32x32x16_bf16 with codewords as rows and keys as columns evaluates
-//   v_j = |c_j|^2 - 2 x.c_j + X_up = |x - c_j|^2 + (X_up - |x|^2),   X_up = |x|^2 rounded up to bf16.
+// Screen.  With mu a point near the middle of the block's codebook, c' = c - mu and n = |c'|^2 + 2 mu.c',
+// v_mfma_f32_32x32x16_bf16 with codewords as rows and keys as columns evaluates
+//   v_j = n_j - 2 x.c'_j + X_up = |x - c_j|^2 + (X_up - |x - mu|^2),   X_up = |x - mu|^2 rounded up to bf16.
 // Every fp32 number enters as a sum of bf16 parts (RNE, each the rounding of what the previous left):
-//   bf16 keys (and fp32 keys whose low halves are all zero):  x . (c_hi + c_mid + c_lo), exact products;
-//   other keys:  x_hi (c_hi + c_mid) + x_mid c_hi, which leaves out at most 3 2^-18 |x||c| per product;
-//   block dims 1 and 2, any key:  the six products down to 2^-18, which leave out less than 2^-25 |x||c|;
-//   |c|^2 in three parts against 1, X_up against 1.
+//   bf16 keys (and fp32 keys whose low halves are all zero):  x . (c'_hi + c'_mid + c'_lo), exact products;
+//   block dims 1 and 2, any key:  the six products down to 2^-18, which leave out less than 2^-25 |x||c'|;
+//   other keys, with x' = x - mu in place of x and n = |c'|^2:  x'_hi (c'_hi + c'_mid) + x'_mid c'_hi, which
+//   leaves out at most 3 2^-18 |x'||c'| per product;
+//   n in three parts against 1, X_up against 1.
 // That is 3 bd + 4 (6 bd + 4) of the K slots: one MFMA for block dims up to 4, two for 8, four for 16.
-// v_j >= 0 up to rounding, so its bits order as a signed int.
+// v_j >= 0 up to rounding, so its bits order as a signed int.  (bf16 keys keep their own bits, as x - mu
+// is no bf16 number.)  No product is larger than |x||c'|, so an offset that keys and codewords share, as K
+// projections have per channel, weighs on the error bound once and not squared.
 //
 // What it replaces and why.  The fp32 form (v_mfma_f32_16x16x4f32, K = bd + 2 padded to 8) spent 64
 // matrix-core cycles per 256 distances and three VALU instructions per distance on the lane's two
@@ -21,27 +25,43 @@
 // a group on each of a key's two lanes.
 //
 // Measured, one MI355X, the fp32 screen / exact scan before -> this kernel: 262,144 bf16 keys of head_dim
-// 128 at block_dim 4, 256 codewords: 625 -> 164 us (77 MB, 15 us at a copy's rate: VALU issue bounds it,
-// 288 VALU instructions per 32 keys and block at 73 % issue, the matrix cores 13 % busy); 65,536 fp32
-// keys at 4,096 codewords of dim 4: 1,448 -> 375 us; a 64-sequence decode step's append: unchanged,
-// 11 us.
+// 128 at block_dim 4, 256 codewords: 631 -> 184 us (77 MB, 15 us at a copy's rate: VALU issue bounds it,
+// 283 VALU instructions per 32 keys and block in 68 % of the issue slots, the matrix cores 15 % busy);
+// 65,536 fp32 keys at 4,096 codewords of dim 4, with the dequantize's 26: 1,434 -> 404 us (VALU 82 %,
+// matrix cores 32 %); a 64-sequence decode step's append: 13.4 -> 13.1 us with the call.
+// Keys and codewords that share an offset of 0, 10, 30 and 100 standard deviations, bf16, 8 heads: 8,192 rows
+// at 256 codewords of dim 4: 59, 61, 76 and 205 us (the fp32 screen 168, 204, 257 and 439; with |x|^2 in this
+// screen's bound 54, 94, 546 and 977); 4,096 rows at 4,096 codewords: 205, 304, 718 and 1,035 (the exact scan
+// 735).  Slower than what they replaced: codebooks past 256 codewords around the last offset, or that hold
+// every codeword twice (1.1 to 1.4 times, at 300 codewords 1.8), and block dims 9 and 10 for at most 128 keys
+// with an offset (32 against 16 us).
 //
-// Error bound.  P_j = (|x| + |c_j|)^2.  The terms of v_j pass through at most as many
-// roundings (any order, even truncation) of partial sums of at most 1.02 P_j, |c_j|^2 carries the
-// bd roundings of the reference's own norm, and the parts left out add 1.53 2^-18 P_j (2^-24):
-// |v_j - (|x - c_j|^2 + X_up - |x|^2)| <= A P_j.  The reference's chain r_j is within g P_j of
-// |x - c_j|^2, g = 1.001 (bd + 2) 2^-23.  With |c_j| <= |x| + |x - c_j|, P_j <= 6 |x|^2 + 3 |x - c_j|^2.
-// The reference's winner j* has sqrt(r_j*) <= sqrt(r_m) for the screen's minimum m, and a correctly
-// rounded sqrt merges values at most 2^-21 apart, so with S = max(v_m - (X_up - |x|^2), 0) and
-// B = A + g,
-//   v_j* <= v_m + 2^-20 S + 2 B (6 |x|^2 + 3 (1.01 S + 64 B |x|^2))
-//        <= v_m + (2^-20 + 6.2 B) S + 12.6 B |x|^2         (B < 2^-15).
+// Error bound.  d_j = |x - c_j|, y = |x - mu|, m = |mu|; |c'_j| <= y + d_j.  The terms of v_j pass through
+// at most as many roundings (any order, even truncation) of partial sums of at most
+// 1.02 (|c'|^2 + 2 (m + |x|) |c'| + 1.01 y^2); n carries 2 bd roundings of its own, c' and x' one each, and
+// the parts left out add L |x||c'|, L = 6.16 2^-18 (0 for keys exact in one part).  So with
+// A = 1.02 terms 2^-23 + (2 bd + 2) 2^-24,
+//   |v_j - (d_j^2 + X_up - y^2)| <= A (2.51 y^2 + 3 d_j^2 + 2 (m + |x|) (y + d_j)) + L |x| (y + d_j),
+// and for two-part keys the same with y for |x| and 0 for m.
+// The reference's chain r_j = ((-2x.c_j) + |x|^2) + |c_j|^2 rounds its product's bd steps at most at
+// 2 |x||c_j|, the first sum at d_j^2 + |c_j|^2 and the second at d_j^2, and |c_j|^2 carries bd roundings;
+// the roundings of |x|^2 are the same for every j.  Beside those it is within G_j of d_j^2, with
+// g = 1.01 2^-24 and |c_j| <= |x| + d_j,
+//   G_j <= g (2 bd |x||c_j| + (bd + 1) |c_j|^2 + 2 d_j^2) <= g ((3.13 bd + 1.07) |x|^2 + (33 bd + 19) d_j^2).
+// The reference's winner j* has sqrt(r_j*) <= sqrt(r_m) (negative r: 0, which adds no more than the
+// roundings of |x|^2, at most bd g |x|^2) for the screen's minimum m, and a correctly rounded sqrt merges
+// values at most 2^-21 apart, so with S = max(v_m - (X_up - y^2), 0), both d_j*^2 and d_m^2 are at most
+// Q = 1.03 S + 20 (A + L + 2 g (3.13 bd + 1.07)) (|x|^2 + y^2), and
+//   v_j* <= v_m + 5.02 A y^2 + 2 g (3.13 bd + 1.07) |x|^2 + (6 A + 2 g (33 bd + 19) + 2^-20) Q
+//               + (4 A m + (4 A + 2 L) |x|) sqrt(2 (y^2 + Q)),   m <= |x| + y;
+// where mu is 0 (y = |x|), the last term is at most (4 A + 2 L) (1.4143 |x|^2 + 0.7072 Q).
 // thr adds 2^-17 relative for the tag bits (at most 2^-18 of v_m) and 2^-100 for underflow.  Every
 // codeword that can win has v <= thr, so when one group alone reaches thr the winner is in it.
 // Otherwise (and for keys or codewords whose squares pass 2^120 or are not finite, and when two
-// candidates' distances are too close for their square roots to be told apart) the wave evaluates
-// every codeword of the block for that key.  The code is therefore the reference's, whatever the
-// matrix core's rounding order.
+// candidates' distances are too close for their square roots to be told apart) every codeword of the
+// block is evaluated for that key: such pairs go to a list that the whole workgroup scans at its end, 16
+// lanes a pair, or, where a block leaves many, to a scan of the block from LDS.  The code is
+// therefore the reference's, whatever the matrix core's rounding order.
 #include "ssq_encode_math.h"
 
 #include <string.h>
@@ -76,14 +96,23 @@ constexpr int kMaxLightTile = 128;
 
 enum { kKeyBf16 = 0, kKeyF16 = 1, kKeyF32 = 2 };
 
+// factors of the file comment's threshold
+struct ScreenBound {
+    float s, a, x;    // S, |x - mu|^2, |x|^2
+    float qa, qs, qx;  // |x - mu|^2, S, |x|^2 inside the square root that bounds |x - mu| + |x - c|
+    float m, n;       // |mu|, |x| (two-part keys: |x - mu|) times that root
+    float cs, cx;     // S, |x|^2 where mu is 0
+};
+
 struct TileParams {
     ssq_encode_args a;
-    float ex[2], es[2];  // thr's |x|^2 and S factors: [0] keys exact in one bf16 part, [1] two-part keys
+    ScreenBound bound[2];  // [0] keys exact in one bf16 part, [1] two-part keys
     int nbc;             // light blocks per workgroup chunk
     int n_light, chunks, fold;
     int xg, groups;      // key groups per (sequence, KV head), and in all
     int row_codes;       // 1: one chunk holds every light block and code rows take 16-byte stores
     int vec;             // 1: codeword rows are aligned for vector loads
+    int center;          // 0: mu is 0
     int pieces;          // 16-byte pieces per key row where rows load whole (a power of two), else 0
     uint8_t light[kMaxLightTile];  // light (VQ-coded) block ids, ascending
 };
@@ -99,19 +128,34 @@ struct TileShape {
 };
 constexpr int slot_dwords(int bdp, bool raw16) { return raw16 ? bdp / 2 : bdp; }
 
-// (key, block) pairs a workgroup can put off to its end (the full scans); more are scanned at once
-constexpr int kOpenCap = 512;
+// (key, block) pairs that a workgroup can put off: to its end, or (256 codewords) until kOpenFlush are
+// waiting after a block.  A block that leaves more than open_block of its 512 keys open is scanned for
+// all of them at once (scan_block): one pair costs 1.6 times as much on the list, where a lane reads each
+// codeword from memory, at 256 codewords, 3.5 at 4,096 and 7 at 16,384.  Once two blocks and at
+// least half of those so far failed (of a chunk of at most 8 blocks: the first one, with more than
+// kOpenMost open), the screen ends and the rest are scanned.
+constexpr int kOpenCap = 1024;
+constexpr int kOpenFlush = 512;
+__device__ __forceinline__ int open_block(int nc) { return nc <= 256 ? 256 : nc <= 8192 ? 128 : 64; }
+constexpr int kOpenMost = kTileKeys / 2;
 
-// LDS: operands [2][kOps] | (one stage only: records [2][kRecs]) | bad [nbc], two-part flag, open
-//      count | slot of block [128] | heavy blocks [128] | open pairs [kOpenCap] u16 | (under a
-//      metric: E_b [nbc][BDP][BDP]) | keys [nbc + 1][kKeyRow][slot dwords] (the last slot takes
-//      the dims of other chunks and of heavy blocks where rows load whole; block dims 9 and 10 are
-//      always gathered and have none)
+// mu costs a small call up to 1 us and saves it little: few open pairs have the whole workgroup (block
+// dims 9 and 10, whose scans are the longest, take it at every size)
+constexpr int kCenterKeys = 64;
+
+// LDS: operands [2][kOps] | (one stage only: records [2][kRecs]) | bad [nbc] (1: not finite, 4: mu is not 0, 2: failed), two-part flag, open
+//      count, failed [2], a block's open count [3], unused | mu [nbc][BDP] | decided keys
+//      [nbc][kTileWaves] | slot of block [128] | heavy blocks [128] | open pairs [kOpenCap] u16 | (under a
+//      metric: E_b [nbc][BDP][BDP]) | keys [nbc (+ 1)][kKeyRow][slot dwords]: where rows load whole, the
+//      last slot takes the dims of other chunks and of heavy blocks (a chunk of every dim has none of
+//      them, and block dims 9 and 10 are always gathered)
 template <int BDP, bool WIDE>
 size_t tile_smem(int nbc, bool raw16, const ssq_encode_args& a) {
     using Sh = TileShape<BDP, WIDE>;
-    const size_t dw = 2 * (size_t)Sh::kOps + 2 * (size_t)Sh::kRecs + (size_t)((nbc + 5) & ~3) + 64 + kOpenCap / 2;
-    return (dw + (a.metric ? (size_t)nbc * BDP * BDP : 0) + (size_t)(nbc + (BDP < 16 ? 1 : 0)) * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
+    const size_t dw = 2 * (size_t)Sh::kOps + 2 * (size_t)Sh::kRecs + (size_t)((nbc + 11) & ~3) +
+                      (size_t)((nbc * BDP + 3) & ~3) + (size_t)nbc * kTileWaves + 64 + kOpenCap / 2;
+    const int slots = nbc + (BDP < 16 && nbc * BDP != a.head_dim ? 1 : 0);
+    return (dw + (a.metric ? (size_t)nbc * BDP * BDP : 0) + (size_t)slots * kKeyRow * slot_dwords(BDP, raw16)) * 4 + 16;
 }
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
@@ -285,15 +329,21 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     u32a* recs = ops + 2 * Sh::kOps;
     u32a* bad = recs + 2 * Sh::kRecs;
     u32a* two_part = bad + p.nbc;
+    uint32_t* badA = tile_lds + 2 * Sh::kOps + 2 * Sh::kRecs;
     uint32_t* n_open = tile_lds + 2 * Sh::kOps + 2 * Sh::kRecs + p.nbc + 1;
-    uint8_t* blkslot = reinterpret_cast<uint8_t*>(bad + ((p.nbc + 5) & ~3));
+    uint32_t* failed = n_open + 1;  // [parity of the block]
+    uint32_t* n_blk = failed + 2;   // [block modulo 3]
+    u32a* muL = bad + ((p.nbc + 11) & ~3);
+    u32a* okL = muL + ((p.nbc * BDP + 3) & ~3);
+    uint8_t* blkslot = reinterpret_cast<uint8_t*>(okL + p.nbc * kTileWaves);
     uint8_t* heavyL = blkslot + 128;
     u16a* open_list = reinterpret_cast<u16a*>(heavyL + 128);
     float* metL = reinterpret_cast<float*>(open_list + kOpenCap);  // [nl][BDP][BDP]
     u32a* keysL = reinterpret_cast<u32a*>(open_list + kOpenCap) + (a.metric ? p.nbc * BDP * BDP : 0);
     u32a* mykeys = keysL + (wave * 32) * SD;  // slot j of key m: mykeys + (j * kKeyRow + m) * SD
 
-    for (int j = tid; j <= p.nbc + 1; j += kTileThreads) bad[j] = 0;  // and *two_part, *n_open
+    for (int j = tid; j < p.nbc + 7; j += kTileThreads) bad[j] = 0;  // and *two_part, *n_open, failed, n_blk
+    for (int j = tid; j < p.nbc * kTileWaves; j += kTileThreads) okL[j] = ~0u;
     if (tid < nb) {
         const bool hv = ssq_is_heavy(hm0, hm1, tid);
         const int ho = heavy_ordinal(hm0, hm1, tid);
@@ -306,13 +356,22 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     const int64_t* perm = a.perm + (int64_t)kv * a.perm_sh;
     const float* met = a.metric ? a.metric + (int64_t)kv * a.metric_sh : nullptr;
 
-    if (met) {  // the chunk's diagonal blocks of the metric
+    // Loads whose use comes after the keys': the chunk's diagonal blocks of the metric, and for mu, the mean
+    // of 16 codewords spread over a block's codebook, one dim of them per lane.
+    if (met) {
         for (int i = tid; i < nl * BDP * BDP; i += kTileThreads) {
             const int r = i / BDP % BDP, c = i % BDP;
             const int64_t o = p.light[l0 + i / (BDP * BDP)] * bd;
             metL[i] = r < bd && c < bd ? met[(o + r) * D + o + c] : 0.f;
         }
     }
+    float mc[16];
+    auto load_mean = [&](int i) {
+        const float* cb = cent + (int64_t)p.light[l0 + i / BDP] * nc * bd + min(i % BDP, bd - 1);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) mc[u] = cb[((uint32_t)(u * nc) >> 4) * (uint32_t)bd];
+    };
+    if (p.center && tid < nl * BDP) load_mean(tid);
 
     // output rows of this lane's key, and the row of its elements
     int64_t crow = 0, prow = 0, krow = 0;
@@ -445,7 +504,35 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         }
         wave_sync_lds();
     }
-    if (met) __syncthreads();  // metL
+    if (p.center || met) __syncthreads();  // metL, and bad is cleared
+    // mu: 0 where the codebook is centred already (or not finite)
+    for (int i = tid; p.center && i < nl * BDP; i += kTileThreads) {
+        if (i >= kTileThreads) load_mean(i);
+        const int d = i % BDP;
+        float m = 0.f, q = 0.f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            m += mc[u];
+            q = __builtin_fmaf(mc[u], mc[u], q);
+        }
+        m = d < bd ? m * 0.0625f : 0.f;
+        q = d < bd ? q * 0.0625f : 0.f;
+        float m2 = m * m;
+#pragma unroll
+        for (int o = 1; o < BDP; o <<= 1) {
+            m2 += __shfl_xor(m2, o);
+            q += __shfl_xor(q, o);
+        }
+        m = m2 > 0.25f * q ? m : 0.f;
+        if (met) {  // its image
+            float y = 0.f;
+#pragma unroll
+            for (int c = 0; c < BDP; ++c) y = __builtin_fmaf(metL[i * BDP + c], __shfl(m, (lane & ~(BDP - 1)) + c), y);
+            m = y;
+        }
+        muL[i] = __float_as_uint(m);
+        if (m != 0.f) bad[i / BDP] = 4;
+    }
     if (KM == kKeyF32 && met && live) {  // the key blocks' images under the block metric
         low = 0;
         for (int j = half; j < nl; j += 2) {
@@ -467,7 +554,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     if (KM == kKeyF32 && low) *two_part = 1;
     __syncthreads();
     const bool one_part = BDP == 2 || KM == kKeyBf16 || (KM == kKeyF32 && *two_part == 0);
-    const float ex = one_part ? p.ex[0] : p.ex[1], es = one_part ? p.es[0] : p.es[1];
+    const ScreenBound& bound = p.bound[one_part ? 0 : 1];
 
     // A stage's codewords, one per thread: with 1,024-codeword stages every wave builds, with smaller
     // ones the waves take turns.  The rows load two stages ahead; the operand is written at the start
@@ -492,14 +579,26 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     auto store_cw = [&](int it, int j, int st) {
         if (met) to_metric<BDP>(metL + j * BDP * BDP, cw);
         const float cn = norm_p<BDP>(cw);
-        if (!(cn < 0x1.0p120f)) bad[j] = 1;
+        if (!(cn < 0x1.0p120f)) atomicOr(&badA[j], 1u);
+        float c[BDP], n = cn;  // the codeword from mu, and |c|^2 (+ 2 mu.c)
+#pragma unroll
+        for (int d = 0; d < BDP; ++d) c[d] = cw[d];
+        if (__builtin_amdgcn_readfirstlane(bad[j]) & 4) {  // mu is not 0
+            n = 0.f;
+#pragma unroll
+            for (int d = 0; d < BDP; ++d) {
+                const float mu = __uint_as_float(muL[j * BDP + d]);
+                c[d] = cw[d] - mu;
+                n = __builtin_fmaf(__builtin_fmaf(one_part ? 2.0f : 0.0f, mu, c[d]), c[d], n);
+            }
+        }
         uint32_t kd[8 * NM];
 #pragma unroll
         for (int i = 0; i < 8 * NM; ++i) kd[i] = 0;
 #pragma unroll
         for (int d = 0; d < BDP; d += 2) {
             float r0, r1, s0, s1;
-            const uint32_t hw = split2(-2.0f * cw[d], -2.0f * cw[d + 1], r0, r1);
+            const uint32_t hw = split2(-2.0f * c[d], -2.0f * c[d + 1], r0, r1);
             const uint32_t mw = split2(r0, r1, s0, s1), lw = pk_bf16(s0, s1);
             if constexpr (BDP == 2) {
                 kd[0] = kd[2] = kd[5] = hw;
@@ -512,8 +611,8 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
             }
         }
         float r1, u, r2;
-        split2(cn, 0.f, r1, u);
-        kd[kNorm] = split2(cn, r1, u, r2);
+        split2(n, 0.f, r1, u);
+        kd[kNorm] = split2(n, r1, u, r2);
         kd[kNorm + 1] = pk_bf16(r2, 1.0f);
         if (WIDE && st * kSc + bcw >= nc) {  // past the codebook's end: 2^126, larger than any threshold
 #pragma unroll
@@ -533,46 +632,123 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
             rec[4 * BDP + (bcw & 3)] = __float_as_uint(cn);
         }
     };
-    // every codeword of block j for key kk of the workgroup, over the lanes of a wave: the reference's
-    // chain, the first index of the smallest sqrt.  A wave busy with it holds the whole workgroup at
-    // the next barrier (it takes longer than a 256-codeword block), so the open pairs wait for the
-    // end, where the lanes share them, and this serves only those past the list's end.
-    auto scan_all = [&](int j, int kk) {
-        u32a* ks = keysL + (j * kKeyRow + kk) * SD;
+    // Codewords n1 + 16 i below n2 of a listed pair on one lane: (sqrt bits, index) of its first minimum,
+    // which order as the reference does.
+    auto scan_pair = [&](int pair, int n1, int n2, auto batch) {
+        constexpr int NB = decltype(batch)::value;  // codewords in flight
+        const int j = pair / kTileKeys;
         uint32_t kwm[SD];
         float xm[BDP];
-        lds_dwords<SD>(ks, kwm);
+        lds_dwords<SD>(keysL + (j * kKeyRow + pair % kTileKeys) * SD, kwm);
         slot_elems<BDP, KM>(kwm, xm);
         const float xmn = norm_p<BDP>(xm);
 #pragma unroll
         for (int d = 0; d < BDP; ++d) xm[d] = -2.0f * xm[d];
-        const int blk = p.light[l0 + j];
-        const float* cb = cent + (int64_t)blk * nc * bd;
-        float be = INFINITY;  // the smallest clamped value, and the first index of its sqrt
+        const float* cb = cent + (int64_t)p.light[l0 + j] * nc * bd;
+        float be = INFINITY;
         uint32_t bn = 0x7FFFFFFFu;
-        constexpr int NB = BDP <= 4 ? 4 : BDP <= 8 ? 2 : 1;
 #pragma unroll 1
-        for (int n0 = lane; n0 < nc; n0 += 64 * NB) {
+        for (int n0 = n1; n0 < n2; n0 += 16 * NB) {
             float c[NB][BDP];
 #pragma unroll
-            for (int i = 0; i < NB; ++i) load_row<BDP>(cb, min(n0 + 64 * i, nc - 1), bd, p.vec, c[i]);
+            for (int u = 0; u < NB; ++u) load_row<BDP>(cb, min(n0 + 16 * u, nc - 1), bd, p.vec, c[u]);
 #pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                if (met) to_metric<BDP>(metL + j * BDP * BDP, c[i]);
+            for (int u = 0; u < NB; ++u) {
+                if (met) to_metric<BDP>(metL + j * BDP * BDP, c[u]);
                 // past the end: the last codeword again, which cannot win over itself
-                take_min(exact_e<BDP>(xm, xmn, c[i], norm_p<BDP>(c[i])), (uint32_t)min(n0 + 64 * i, nc - 1), be, bn);
+                take_min(exact_e<BDP>(xm, xmn, c[u], norm_p<BDP>(c[u])), (uint32_t)min(n0 + 16 * u, nc - 1), be, bn);
             }
         }
-        if (bn == 0x7FFFFFFFu) bn = (uint32_t)lane;  // every value infinite
-        float bf = __builtin_sqrtf(be);
+        if (bn == 0x7FFFFFFFu) bn = (uint32_t)min(n1, nc - 1);  // every value infinite
+        return ((unsigned long long)__float_as_uint(__builtin_sqrtf(be)) << 32) | bn;
+    };
+    auto put_code = [&](int pair, uint32_t n) { keysL[(pair / kTileKeys * kKeyRow + pair % kTileKeys) * SD] = n; };
+    // the list, between two blocks (the whole workgroup): 16 lanes a pair
+    auto scan_list = [&]() {
+        const int n = min((int)__builtin_amdgcn_readfirstlane(*n_open), kOpenCap);
+        for (int i = tid >> 4; i < n; i += kTileThreads / 16) {
+            const int pair = open_list[i];
+            if (bad[pair / kTileKeys] == 2) continue;
+            unsigned long long r =
+                scan_pair(pair, tid & 15, nc, std::integral_constant<int, BDP <= 4 ? 4 : BDP <= 8 ? 2 : 1>{});
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float of = __shfl_xor(bf, o);
-            const uint32_t on = (uint32_t)__shfl_xor((int)bn, o);
-            if (of < bf || (of == bf && on < bn)) { bf = of; bn = on; }
+            for (int o = 8; o > 0; o >>= 1) {
+                const unsigned long long t = ((unsigned long long)(uint32_t)__shfl_xor((int)(r >> 32), o) << 32) |
+                                             (uint32_t)__shfl_xor((int)(uint32_t)r, o);
+                r = t < r ? t : r;
+            }
+            if ((tid & 15) == 0) put_code(pair, (uint32_t)r);
         }
-        if (lane == 0) ks[0] = bn;
-        wave_sync_lds();
+        __syncthreads();
+        if (tid == 0) *n_open = 0;
+    };
+    // Every codeword of block j for its undecided keys (the whole workgroup; the operand buffers' space):
+    // a stage's codewords and norms in LDS, half of them on each of a key's two lanes.
+    auto scan_block = [&](int j) {
+        constexpr int kBuf = kSc / 4 * Sh::kRec;
+        static_assert(kBuf <= Sh::kOps, "a stage's records fit its operand");
+        const int blk = p.light[l0 + j];
+        const float* cb = cent + (int64_t)blk * nc * bd;
+        const uint32_t need = live ? ~(uint32_t)__builtin_amdgcn_readfirstlane(okL[j * kTileWaves + wave]) : 0u;
+        u32a* ks = mykeys + (j * kKeyRow + col) * SD;
+        float m2x[BDP];
+        {
+            uint32_t kw[SD];
+            lds_dwords<SD>(ks, kw);
+            slot_elems<BDP, KM>(kw, m2x);
+        }
+        const float xn = norm_p<BDP>(m2x);
+#pragma unroll
+        for (int d = 0; d < BDP; ++d) m2x[d] = -2.0f * m2x[d];
+        float be = INFINITY;
+        uint32_t bn = (uint32_t)half;  // (every value infinite: the first index)
+        float c[BDP];
+        if (tid < kSc) load_row<BDP>(cb, min(tid, nc - 1), bd, p.vec, c);
+        for (int st = 0; st < nst; ++st) {
+            u32a* buf = ops + (st & 1) * kBuf;
+            if (tid < kSc) {
+                if (met) to_metric<BDP>(metL + j * BDP * BDP, c);
+                u32a* rec = buf + (tid >> 2) * Sh::kRec;
+#pragma unroll
+                for (int d = 0; d < BDP; ++d) rec[(tid & 3) * BDP + d] = __float_as_uint(c[d]);
+                rec[4 * BDP + (tid & 3)] = __float_as_uint(norm_p<BDP>(c));
+                if (st + 1 < nst) load_row<BDP>(cb, min((st + 1) * kSc + tid, nc - 1), bd, p.vec, c);
+            }
+            __syncthreads();
+            if (need) {
+                // (past the end: the last codeword again, which cannot win over itself)
+                constexpr int NR = BDP <= 4 ? 2 : 1;  // records whose distances are computed before their tests
+                const int n_rec = (min(kSc, nc - st * kSc) + 3) / 4, mid = (n_rec / 2 + NR - 1) / NR * NR;
+                const int g1 = half ? n_rec : mid;
+                for (int g = half ? mid : 0; g < g1; g += NR) {
+                    float e[4 * NR];
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) {
+                        uint32_t rec[Sh::kRec];
+                        lds_dwords<Sh::kRec>(buf + (g + r) * Sh::kRec, rec);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float v = m2x[0] * __uint_as_float(rec[i * BDP]);
+#pragma unroll
+                            for (int d = 1; d < BDP; ++d) v = __builtin_fmaf(m2x[d], __uint_as_float(rec[i * BDP + d]), v);
+                            v = __builtin_fmaf(xn, 1.0f, v);
+                            e[4 * r + i] = __builtin_fmaf(1.0f, __uint_as_float(rec[4 * BDP + i]), v);
+                        }
+                    }
+                    const int j0 = st * kSc + 4 * g;
+#pragma unroll
+                    for (int i = 0; i < 4 * NR; ++i) take_min(e[i], (uint32_t)min(j0 + i, nc - 1), be, bn);
+                }
+            }
+        }
+        __syncthreads();  // the buffers' last reads
+        if (need) {
+            const float bf = __builtin_sqrtf(be), of = __shfl_xor(bf, 32);
+            const uint32_t on = (uint32_t)__shfl_xor((int)bn, 32);
+            if (of < bf || (of == bf && on < bn)) bn = on;
+            if (half == 0 && ((need >> col) & 1)) ks[0] = bn;
+            wave_sync_lds();
+        }
     };
 
     load_next(0);
@@ -580,19 +756,56 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
     load_next(1);
     __syncthreads();
 
-    for (int j = 0, it = 0; j < nl; ++j) {
-        u32a* ks = mykeys + (j * kKeyRow + col) * SD;
+    int n_fail = 0;
+    for (int j = 0, it = 0, j3 = 0;; ++j, j3 = j3 == 2 ? 0 : j3 + 1) {
+        u32a* ks = mykeys + (max(min(j, nl - 1), 0) * kKeyRow + col) * SD;
         uint32_t kw[SD];
+        lds_dwords<SD>(ks, kw);
+        const uint32_t bj = bad[j], fj = failed[(j & 1) ^ 1];  // (bad[nl] is a word of its own)
+        // What the block before left open.  A wave of this block sets the other flag, and that one again
+        // only after this block's barrier; the count of the next block is cleared meanwhile.
+        const uint32_t fl = __builtin_amdgcn_readfirstlane(fj);
+        if (fl) {  // uniform
+            __syncthreads();
+            if (tid == 0) failed[(j & 1) ^ 1] = 0;
+            if (fl & 3) {
+                ++n_fail;
+                const bool quit = 2 * n_fail >= j && (n_fail >= 2 || ((fl & 2) && nl <= 8));
+                for (int i = j - 1 + tid; i < (quit ? nl : j); i += kTileThreads) bad[i] = 2;
+                if (quit) {
+                    for (int i = j * kTileWaves + tid; i < nl * kTileWaves; i += kTileThreads) okL[i] = 0;
+                    break;
+                }
+            }
+            if constexpr (!WIDE) {
+                if (fl & 4) {
+                    __syncthreads();  // bad[j - 1]
+                    scan_list();
+                    __syncthreads();  // *n_open
+                }
+            }
+        }
+        if (j >= nl) break;
+        if (tid == 0) n_blk[j3 == 2 ? 0 : j3 + 1] = 0;
         float x[BDP];
-        float xn = 0.f, dlt = 0.f;
+        float xn = 0.f, an = 0.f, dlt = 0.f;
+        const bool off = __builtin_amdgcn_readfirstlane(bj) & 4;  // mu is not 0
         v8bf kb[NM];
         if (live) {
             // the key's operand: [hi, hi, hi or mid, 1, 1, 1, X_up]
-            lds_dwords<SD>(ks, kw);
             slot_elems<BDP, KM>(kw, x);
             xn = norm_p<BDP>(x);
-            const uint32_t xu = (__float_as_uint(xn) + 0xFFFFu) & 0xFFFF0000u;
-            dlt = __uint_as_float(xu) - xn;
+            float xc[BDP];
+#pragma unroll
+            for (int d = 0; d < BDP; ++d) xc[d] = x[d];
+            an = xn;
+            if (off) {
+#pragma unroll
+                for (int d = 0; d < BDP; ++d) xc[d] = x[d] - __uint_as_float(muL[j * BDP + d]);
+                an = norm_p<BDP>(xc);
+            }
+            const uint32_t xu = (__float_as_uint(an) + 0xFFFFu) & 0xFFFF0000u;
+            dlt = __uint_as_float(xu) - an;
             uint32_t kd[8 * NM];
 #pragma unroll
             for (int i = 0; i < 8 * NM; ++i) kd[i] = 0;
@@ -613,7 +826,7 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                     hw = third = kw[d / 2];
                 } else {
                     float r0, r1;
-                    hw = split2(x[d], x[d + 1], r0, r1);
+                    hw = split2(one_part ? x[d] : xc[d], one_part ? x[d + 1] : xc[d + 1], r0, r1);
                     third = one_part ? hw : pk_bf16(r0, r1);
                 }
                 kd[d / 2] = hw;
@@ -701,12 +914,19 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                 pair32((m1 & -32) | ((m1 & 15) << 1) | half, pa, pb);
                 const int pk = min(pa, pb);
                 const float mt = fmaxf(__int_as_float(pk & -32), 0.f) * (1.0f + 0x1.0p-17f);
-                const float thr = mt + es * fmaxf(mt - dlt, 0.f) + ex * xn + 0x1.0p-100f;
+                const float sm = fmaxf(mt - dlt, 0.f);
+                float thr = mt + (bound.cs * sm + bound.cx * xn) + 0x1.0p-100f;
+                if (off) {
+                    const float root = __builtin_amdgcn_sqrtf(bound.qa * an + (bound.qs * sm + bound.qx * xn));
+                    const float xr = __builtin_amdgcn_sqrtf(one_part ? xn : an), y = __builtin_amdgcn_sqrtf(an);
+                    thr = mt + (bound.s * sm + bound.a * an + bound.x * xn) +
+                          root * (bound.n * xr + bound.m * (xr + y)) + 0x1.0p-100f;  // m <= |x| + y
+                }
                 const uint64_t b1 = __builtin_amdgcn_ballot_w64(__int_as_float(m1 & -32) <= thr);
                 const uint64_t b2 = __builtin_amdgcn_ballot_w64(__int_as_float(m2 & -32) <= thr);
                 const uint64_t fin = __builtin_amdgcn_ballot_w64(xn < 0x1.0p120f);
                 uint32_t ok = (uint32_t)fin & (uint32_t)(b1 ^ (b1 >> 32)) & ~(uint32_t)(b2 | (b2 >> 32));
-                if (__builtin_amdgcn_readfirstlane(bad[j])) ok = 0;
+                if (__builtin_amdgcn_readfirstlane(bad[j]) & 1) ok = 0;
                 float m2x[BDP];
 #pragma unroll
                 for (int d = 0; d < BDP; ++d) m2x[d] = -2.0f * x[d];
@@ -759,67 +979,49 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
                 // the code takes the place of the block's key elements
                 if (mine && ((ok >> col) & 1)) ks[0] = (uint32_t)(first + best[0].n);
                 const uint32_t todo = ~ok;
-                if (todo) {  // rare: to the list for the end; what does not fit there is scanned here
+                if (todo) {  // to the list, unless the block fails (scan_block then serves it)
+                    const int n = __popc(todo);
                     int at = 0;
-                    if (lane == 0) at = (int)atomicAdd(n_open, (uint32_t)__popc(todo));
+                    if (lane == 0) {
+                        okL[j * kTileWaves + wave] = ok;
+                        const int c = (int)atomicAdd(&n_blk[j3], (uint32_t)n) + n;
+                        at = c > open_block(nc) ? kOpenCap : (int)atomicAdd(n_open, (uint32_t)n);
+                        if (at + n > kOpenCap) atomicOr(&failed[j & 1], c > kOpenMost ? 3u : 1u);
+                        else if (!WIDE && at + n > kOpenFlush) atomicOr(&failed[j & 1], 4u);
+                    }
                     at = __builtin_amdgcn_readfirstlane(at);
                     const int pos = at + __popc(todo & ((1u << col) - 1u));
                     if (half == 0 && ((todo >> col) & 1) && pos < kOpenCap)
                         open_list[pos] = (uint16_t)(j * kTileKeys + wave * 32 + col);
-                    if (at + __popc(todo) > kOpenCap) {
-                        wave_sync_lds();
-                        for (uint32_t t = todo; t; t &= t - 1)
-                            if (at++ >= kOpenCap) scan_all(j, wave * 32 + __builtin_ctz(t));
-                    }
                 }
                 wave_sync_lds();
             }
             __syncthreads();
         }
     }
-    // The pairs put off, published by the loop's last barrier: 16 lanes per 256 codewords of a pair,
-    // 16 codewords a lane; (sqrt bits, index) pairs meet in a 64-bit LDS minimum, which orders them as
-    // the reference does (the operand buffers' space).
+    if (n_fail) {
+        __syncthreads();
+        for (int j = 0; j < nl; ++j)
+            if (__builtin_amdgcn_readfirstlane(bad[j]) == 2) scan_block(j);
+    }
+    // The pairs on the list (published by the loop's last barrier; those of failed blocks are done): 16
+    // lanes per 256 (block dims 9 and 10: 64) codewords of a pair; the results meet in a 64-bit LDS
+    // minimum (the operand buffers' space).
     const int n_put = nl > 0 ? min((int)__builtin_amdgcn_readfirstlane(*n_open), kOpenCap) : 0;
     if (n_put) {
         unsigned long long* res = reinterpret_cast<unsigned long long*>(tile_lds);
         if (tid < n_put) res[tid] = ~0ull;
         __syncthreads();
-        const int parts = (nc + 255) / 256;
+        const int part = BDP == 16 ? 64 : 256, parts = (nc + part - 1) / part;
         for (int i = tid >> 4; i < n_put * parts; i += kTileThreads / 16) {
-            const int en = i / parts, n1 = (i - en * parts) * 256 + (tid & 15);
-            const int j = open_list[en] / kTileKeys;
-            uint32_t kwm[SD];
-            float xm[BDP];
-            lds_dwords<SD>(keysL + (j * kKeyRow + open_list[en] % kTileKeys) * SD, kwm);
-            slot_elems<BDP, KM>(kwm, xm);
-            const float xmn = norm_p<BDP>(xm);
-#pragma unroll
-            for (int d = 0; d < BDP; ++d) xm[d] = -2.0f * xm[d];
-            const int blk = p.light[l0 + j];
-            const float* cb = cent + (int64_t)blk * nc * bd;
-            float be = INFINITY;
-            uint32_t bn = 0x7FFFFFFFu;
-            constexpr int NB = BDP <= 4 ? 16 : BDP <= 8 ? 4 : 1;
-#pragma unroll 1
-            for (int n0 = n1; n0 < n1 + 256; n0 += 16 * NB) {
-                float c[NB][BDP];
-#pragma unroll
-                for (int u = 0; u < NB; ++u) load_row<BDP>(cb, min(n0 + 16 * u, nc - 1), bd, p.vec, c[u]);
-#pragma unroll
-                for (int u = 0; u < NB; ++u) {
-                    if (met) to_metric<BDP>(metL + j * BDP * BDP, c[u]);
-                    take_min(exact_e<BDP>(xm, xmn, c[u], norm_p<BDP>(c[u])), (uint32_t)min(n0 + 16 * u, nc - 1), be, bn);
-                }
-            }
-            if (bn == 0x7FFFFFFFu) bn = (uint32_t)min(n1, nc - 1);  // every value infinite
-            atomicMin(&res[en], ((unsigned long long)__float_as_uint(__builtin_sqrtf(be)) << 32) | bn);
+            const int en = i / parts, n1 = (i - en * parts) * part;
+            const int pair = open_list[en];
+            if (bad[pair / kTileKeys] == 2) continue;
+            atomicMin(&res[en], scan_pair(pair, n1 + (tid & 15), n1 + part,
+                                          std::integral_constant<int, BDP <= 4 ? 16 : BDP <= 8 ? 4 : 1>{}));
         }
         __syncthreads();
-        if (tid < n_put) {
-            const int j = open_list[tid] / kTileKeys;
-            keysL[(j * kKeyRow + open_list[tid] % kTileKeys) * SD] = (uint32_t)res[tid];
-        }
+        if (tid < n_put && bad[open_list[tid] / kTileKeys] != 2) put_code(open_list[tid], (uint32_t)res[tid]);
         __syncthreads();
     }
     if (!live) return;
@@ -888,6 +1090,7 @@ int launch_tile(TileParams& tp, hipStream_t st) {
     tp.fold = ssq_encode_fold(&a, kTileKeys);
     const int64_t n_keys = tp.fold ? (int64_t)a.batch * a.seq_len : a.seq_len;
     const int64_t xg = (n_keys + kTileKeys - 1) / kTileKeys;
+    tp.center = n_keys > kCenterKeys || BDP == 16;
     const int64_t groups = xg * (tp.fold ? a.num_kv_heads : (int64_t)a.batch * a.num_kv_heads);
     // Smaller chunks of blocks until the workgroups fill the chip: a few keys (a decode step's
     // append) take one block per workgroup.  Past 256 codewords a block is long, so the chunks
@@ -945,13 +1148,23 @@ int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st) {
     tp.a = *a;
     const int bd = a->block_dim;
     for (int two = 0; two < 2; ++two) {  // the bound of the file comment, rounded up
-        const double gr = 1.001 * (bd + 2) * 0x1.0p-23;
         const int terms = (bd <= 2 ? 6 : 3) * bd + 4;
-        const double left = bd <= 2 ? 0x1.0p-24 : two ? 1.53 * 0x1.0p-18 : 0.0;
-        const double A = 1.02 * terms * 0x1.0p-23 + bd * 0x1.0p-24 + left;
-        const double B = A + gr;
-        tp.ex[two] = (float)(12.6 * B * 1.001);
-        tp.es[two] = (float)((0x1.0p-20 + 6.2 * B) * 1.001);
+        const double al = 1.02 * terms * 0x1.0p-23 + (2 * bd + 2) * 0x1.0p-24;
+        const double left = bd <= 2 ? 0x1.0p-23 : two ? 6.16 * 0x1.0p-18 : 0.0;
+        const double g = 1.01 * 0x1.0p-24, gx = 2 * g * (3.13 * bd + 1.07), gd = 2 * g * (33 * bd + 19);
+        const double near = 6 * al + gd + 0x1.0p-20, k = 20 * (al + left + gx), up = 1.002;
+        ScreenBound& b = tp.bound[two];
+        b.s = (float)(1.03 * near * up);
+        b.a = (float)((5.02 * al + near * k) * up);
+        b.x = (float)((gx + near * k) * up);
+        b.qa = (float)(2 * (1 + k) * up);
+        b.qs = (float)(2.06 * up);
+        b.qx = (float)(2 * k * up);
+        b.m = (float)(bd > 2 && two ? 0.0 : 4 * al * up);
+        b.n = (float)((4 * al + 2 * left) * up);
+        const double cn = 4 * al + 2 * left;  // |x| sqrt(2 (|x|^2 + Q)) <= 1.4143 |x|^2 + 0.7072 Q
+        b.cs = (float)(1.03 * (near + 0.7072 * cn) * up);
+        b.cx = (float)((5.02 * al + gx + 1.4143 * cn + 2 * k * (near + 0.7072 * cn)) * up);
     }
     for (int blk = 0; blk < a->n_blocks; ++blk) {
         const bool heavy = blk < 64 ? ((a->heavy_mask[0] >> blk) & 1) : ((a->heavy_mask[1] >> (blk - 64)) & 1);
@@ -960,10 +1173,10 @@ int ssq_encode_tile_run(const ssq_encode_args* a, hipStream_t st) {
     const int64_t al = bd == 2 ? 8 : 16;
     tp.vec = (bd == 2 || bd == 4 || bd == 8 || bd == 16) && (uintptr_t)a->cent % al == 0 && (a->cent_sh * 4) % al == 0;
     const bool wide = a->n_centroids > 256;
+    SSQ_UNSUPPORTED(!wide || (bd >= 3 && bd <= 8), "MFMA encode past 256 codewords needs block_dim 3 to 8");
     const int bdp = bd <= 2 ? 2 : bd <= 4 ? 4 : bd <= 8 ? 8 : 16;
     switch (bdp * 2 + (wide ? 1 : 0)) {
         case 4: return launch_tile_keys<2, false>(tp, st);
-        case 5: return launch_tile_keys<2, true>(tp, st);
         case 8: return launch_tile_keys<4, false>(tp, st);
         case 9: return launch_tile_keys<4, true>(tp, st);
         case 16: return launch_tile_keys<8, false>(tp, st);

@@ -122,11 +122,46 @@ def test_tile_heavy_pages_metric_and_repeated_dims(nc):
     assert torch.equal(pages[0], pages[1])
 
 
+@pytest.mark.parametrize("nc,bd", [(256, 4), (256, 1), (256, 10), (700, 4), (1500, 3), (600, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_tile_offsets(nc, bd, dtype):
+    """Keys and codewords that share an offset per dim, up to where rounding hides the differences (every
+    pair on the list, which fills at each block), one that only the keys have, and one that only half
+    of the codewords have."""
+    D = {3: 48, 10: 80}.get(bd, 64)
+    _, perm, cent = _codec(D, bd, nc, 2, nc + bd)
+    n = 1111 if nc == 256 else 2000
+    for i, (off, cut) in enumerate(((0.7, 1.0), (10.0, 1.0), (300.0, 1.0), (5.0, 0.0), (20.0, 0.5))):
+        g = torch.Generator().manual_seed(i)
+        ch = torch.randn(D, generator=g).sign() * off * (1 + torch.rand(D, generator=g))
+        keys = torch.randn(1, 2, n, D, generator=g) + ch
+        c = cent.clone()
+        c[:, :, :int(nc * cut)] += ch.to(DEV)[perm].view(D // bd, 1, bd)
+        assert nc == 256 or _screened(keys, c)
+        _both(keys.to(dtype).to(DEV), perm, c)
+    E = (torch.eye(D) + 0.2 * torch.randn(D, D, generator=g)).to(DEV)
+    _both(keys.to(dtype).to(DEV), perm, c, metric=E)
+
+
 def _offset_problem(n, H, D, bd, nc, dtype, off):
     g = torch.Generator(device=DEV).manual_seed(1)
     perm = torch.randperm(D, generator=g, device=DEV)
     cent = torch.randn(H, D // bd, nc, bd, generator=g, device=DEV) + off
     return (torch.randn(1, H, n, D, generator=g, device=DEV) + off).to(dtype), perm, cent
+
+
+@pytest.mark.parametrize("nc,dtype,n", [(256, torch.float16, 4096), (256, torch.bfloat16, 4096),
+                                        (4096, torch.float32, 2048), (4096, torch.bfloat16, 2048)])
+def test_tile_time_at_an_offset(nc, dtype, n):
+    """An offset of ten standard deviations that keys and codewords share costs at most twice the centred
+    call (1.05 to 1.5 times; a screen whose bound grows with |x|^2, 1.8 to 13 times), and 30 no more than
+    twice the exact scan past 256 codewords, five times the centred call at 256 (1.3; 10 to 17)."""
+    base = time_us(lambda a=_offset_problem(n, 8, 128, 4, nc, dtype, 0.0): hip_ops.encode(*a))
+    ten = time_us(lambda a=_offset_problem(n, 8, 128, 4, nc, dtype, 10.0): hip_ops.encode(*a))
+    far = _offset_problem(n, 8, 128, 4, nc, dtype, 30.0)
+    thirty = time_us(lambda: hip_ops.encode(*far))
+    limit = 5 * base if nc == 256 else 2 * time_us(lambda: hip_ops.encode(*far, kernel=1))
+    assert ten < 2 * base and thirty < limit, (base, ten, thirty, limit)
 
 
 @pytest.mark.parametrize("n,H,D,bd,nc", [(1024, 1, 128, 2, 300), (2048, 8, 128, 1, 1024), (8, 8, 128, 4, 65535)])
