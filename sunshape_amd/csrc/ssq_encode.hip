@@ -152,8 +152,8 @@ extern "C" int ssq_encode(const ssq_encode_args* a, void* stream) {
         SSQ_REQUIRE((uintptr_t)a->codes % cw == 0, "%d-bit codes must be %d-byte aligned", 8 * cw, cw);
         // The screen stages every codebook once per 512 keys of a KV head and folds its groups, which for few
         // keys, and up to about 2^24 (key, block, codeword) triples, costs more than the exact scan split
-        // over lanes: bf16 keys of head_dim 128 over 8 heads, 64 rows at 4,096 codewords of dim 4 (2^23)
-        // 18 us on the scan and 34 on the screen, 8 at 65,535 (2^27) 215 and 454.  Codebooks of dims 1 and 2
+        // over lanes: bf16 keys of head_dim 128, 8 heads, 8 rows each at 4,096 codewords of dim 4 (2^23)
+        // 18 us on the scan and 34 on the screen, at 65,535 (2^27) 215 and 454.  Codebooks of dims 1 and 2
         // stay on the scan: many codewords then lie within the screen's bound of the nearest, which leaves
         // most pairs to a scan of its own (2,048 keys at 1,024 codewords of dim 1: 303 us on the scan, 612
         // on the screen; 4,096 at 1,024 of dim 2, 323 and 136 when centred, 590 with an offset of 30 standard
