@@ -33,8 +33,8 @@
 // at 256 codewords of dim 4: 59, 61, 76 and 205 us (the fp32 screen 168, 204, 257 and 439; with |x|^2 in this
 // screen's bound 54, 94, 546 and 977); 4,096 rows at 4,096 codewords: 205, 304, 718 and 1,035 (the exact scan
 // 735).  Slower than what they replaced: codebooks past 256 codewords around the last offset, or that hold
-// every codeword twice (1.1 to 1.4 times, at 300 codewords 1.8), and block dims 9 and 10 for at most 128 keys
-// with an offset (32 against 16 us).
+// every codeword twice (1.1 to 1.4 times, at 300 codewords 1.8), and block_dim 1 for at most 128 keys (10 to
+// 35 %, 1 to 5 us).
 //
 // Error bound.  d_j = |x - c_j|, y = |x - mu|, m = |mu|; |c'_j| <= y + d_j.  The terms of v_j pass through
 // at most as many roundings (any order, even truncation) of partial sums of at most
@@ -647,8 +647,20 @@ __global__ __launch_bounds__(kTileThreads) void k_encode_tile(const TileParams p
         const float* cb = cent + (int64_t)p.light[l0 + j] * nc * bd;
         float be = INFINITY;
         uint32_t bn = 0x7FFFFFFFu;
+        bool in_lds = false;
+        if constexpr (!WIDE) {  // a chunk of at most two blocks (a few keys) still has their records
+            in_lds = nl <= 2;
+            const u32a* rj = recs + (j & 1) * Sh::kRecs;
+            for (int n = n1; in_lds && n < n2; n += 16) {
+                const u32a* rec = rj + (n >> 2) * Sh::kRec;
+                float c[BDP];
+#pragma unroll
+                for (int d = 0; d < BDP; ++d) c[d] = __uint_as_float(rec[(n & 3) * BDP + d]);
+                take_min(exact_e<BDP>(xm, xmn, c, __uint_as_float(rec[4 * BDP + (n & 3)])), (uint32_t)n, be, bn);
+            }
+        }
 #pragma unroll 1
-        for (int n0 = n1; n0 < n2; n0 += 16 * NB) {
+        for (int n0 = in_lds ? n2 : n1; n0 < n2; n0 += 16 * NB) {
             float c[NB][BDP];
 #pragma unroll
             for (int u = 0; u < NB; ++u) load_row<BDP>(cb, min(n0 + 16 * u, nc - 1), bd, p.vec, c[u]);
