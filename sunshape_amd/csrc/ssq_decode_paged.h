@@ -73,7 +73,13 @@ struct SsqCut {
         int most = 0;  // the fullest workgroup's cost with whole sequences
         for (int w = lane; w < n_wg; w += SSQ_WAVE) {
             int c = 0;
-            for (int b = w; b < a.batch; b += n_wg) c += len(a, b) + fixed;
+            for (int b = w; b < a.batch; b += 8 * n_wg) {
+                int l[8];  // loads in flight together
+#pragma unroll
+                for (int u = 0; u < 8; ++u) l[u] = len(a, min(b + u * n_wg, a.batch - 1));
+#pragma unroll
+                for (int u = 0; u < 8; ++u) c += b + u * n_wg < a.batch ? l[u] + fixed : 0;
+            }
             most = max(most, c);
         }
         whole = __builtin_amdgcn_ballot_w64(most > share + kCutWorth * fixed) == 0;
